@@ -41,9 +41,9 @@ constexpr int Q = 27;
 
 struct Kern {
     hipError_t (*collide)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int, int,
-                          int, int, int, hipStream_t);
-    hipError_t (*thermal)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int, int,
                           int, int, hipStream_t);
+    hipError_t (*thermal)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int, int,
+                          int, hipStream_t);
     hipError_t (*ghost_fill)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int, int,
                              hipStream_t);
     hipError_t (*bouzidi)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int, int,
@@ -175,10 +175,8 @@ struct EngineCase {
 
 // Work lists of one depth of the engine's recursion (concatenated over cases).
 struct DepthWork {
-    lbk::Work *col = nullptr, *colb = nullptr, *gh = nullptr, *lk = nullptr, *tcol = nullptr, *tcolb = nullptr,
-              *tgh = nullptr,
-              *tlk = nullptr;
-    int32_t ncol = 0, ncolb = 0, ngh = 0, nlk = 0, ntcol = 0, ntcolb = 0, ntgh = 0, ntlk = 0;
+    lbk::Work *col = nullptr, *gh = nullptr, *lk = nullptr, *tcol = nullptr, *tgh = nullptr, *tlk = nullptr;
+    int32_t ncol = 0, ngh = 0, nlk = 0, ntcol = 0, ntgh = 0, ntlk = 0;
     int wide = 0, wide_g = 0;
     // force sampling of the cases whose first level runs at this depth:
     // triangle chunks (li = record, item = chunk) and the record indices
@@ -289,12 +287,12 @@ float half_to_float(uint16_t h) {
 
 inline size_t fidx(int64_t b, int k, int c) { return ((size_t)b * Q + k) * NC + c; }
 
-lbk::Work mkwork(int li, int item, int ci, const int32_t* row) {
+lbk::Work mkwork(int li, int item, int ci, const int32_t* row, int32_t flags = 0) {
     lbk::Work w;
     w.li = li;
     w.item = item;
     w.ci = ci;
-    w.pad = 0;
+    w.flags = flags;
     w.nbr_row = row;
     return w;
 }
@@ -524,20 +522,15 @@ int step_level(lb_ctx* c, int li, int64_t j) {
         if (fill) HIPCHK(c, c->k->ghost_fill(las, st, L.wgh, L.n_gchunks, j, storage, 0, c->stream));
         hipEvent_t e1 = nullptr;
         RC(profile_begin(c, L, 0, &e1));
-        HIPCHK(c, c->k->collide(las, st, L.wcol, L.n_int, j, storage, L.wide ? 1 : 0, 0, LB_SCHED_LINEAR,
+        HIPCHK(c, c->k->collide(las, st, L.wcol, L.nb, j, storage, L.wide ? 1 : 0, LB_SCHED_LINEAR,
                                 default_waves(storage), c->stream));
-        HIPCHK(c, c->k->collide(las, st, L.wcol + L.n_int, L.nb - L.n_int, j, storage, L.wide ? 1 : 0, 1,
-                                LB_SCHED_LINEAR, 5, c->stream));
         if (e1) HIPCHK(c, hipEventRecord(e1, c->stream));
         if (L.n_lchunks > 0) HIPCHK(c, c->k->bouzidi(las, st, L.wlk, L.n_lchunks, j, storage, 0, c->stream));
         if (ddf) {
             if (fill) HIPCHK(c, c->k->ghost_fill(las, st, L.wgh, L.n_gchunks, j, storage, 1, c->stream));
             hipEvent_t e2 = nullptr;
             RC(profile_begin(c, L, 1, &e2));
-            HIPCHK(c, c->k->thermal(las, st, L.wcol, L.n_int, j, storage, L.wide_g ? 1 : 0, 0, LB_SCHED_LINEAR,
-                                    c->stream));
-            HIPCHK(c, c->k->thermal(las, st, L.wcol + L.n_int, L.nb - L.n_int, j, storage, L.wide_g ? 1 : 0, 1,
-                                    LB_SCHED_LINEAR, c->stream));
+            HIPCHK(c, c->k->thermal(las, st, L.wcol, L.nb, j, storage, L.wide_g ? 1 : 0, LB_SCHED_LINEAR, c->stream));
             if (e2) HIPCHK(c, hipEventRecord(e2, c->stream));
             if (L.n_lchunks > 0) HIPCHK(c, c->k->bouzidi(las, st, L.wlk, L.n_lchunks, j, storage, 1, c->stream));
         }
@@ -777,7 +770,7 @@ int engine_rebuild(lb_engine* e) {
         W.nfrec = (int32_t)frec[(size_t)d - 1].size();
     }
     for (int d = 1; d <= e->lmax; d++) {
-        std::vector<lbk::Work> col, colb, gh, lk, tcol, tcolb, tgh, tlk;
+        std::vector<lbk::Work> col, colb, gh, lk, tcol, tcolb, tgh, tlk;  // colb, tcolb: boundary blocks, listed last
         DepthWork& W = e->depth[(size_t)d - 1];
         for (size_t i = 0; i < e->cases.size(); i++) {
             const lb_ctx* c = e->cases[i].c;
@@ -790,8 +783,8 @@ int engine_rebuild(lb_engine* e) {
             const bool ddf = c->cfg.ddf_enabled && lev.g[0] != nullptr;
             for (size_t q = 0; q < lev.order_host.size(); q++) {
                 const int32_t b = lev.order_host[q];
-                const lbk::Work w = mkwork(li, b, ci, lev.nbr + (size_t)b * Q);
                 const bool interior = (int32_t)q < lev.n_int;
+                const lbk::Work w = mkwork(li, b, ci, lev.nbr + (size_t)b * Q, interior ? 0 : lbk::WORK_BOUNDARY);
                 (interior ? col : colb).push_back(w);
                 if (ddf) (interior ? tcol : tcolb).push_back(w);
             }
@@ -811,20 +804,18 @@ int engine_rebuild(lb_engine* e) {
             if (lev.wide) W.wide = 1;
             if (lev.wide_g) W.wide_g = 1;
         }
+        col.insert(col.end(), colb.begin(), colb.end());
+        tcol.insert(tcol.end(), tcolb.begin(), tcolb.end());
         RC(eupload(e, &W.col, col));
-        RC(eupload(e, &W.colb, colb));
         RC(eupload(e, &W.gh, gh));
         RC(eupload(e, &W.lk, lk));
         RC(eupload(e, &W.tcol, tcol));
-        RC(eupload(e, &W.tcolb, tcolb));
         RC(eupload(e, &W.tgh, tgh));
         RC(eupload(e, &W.tlk, tlk));
         W.ncol = (int32_t)col.size();
-        W.ncolb = (int32_t)colb.size();
         W.ngh = (int32_t)gh.size();
         W.nlk = (int32_t)lk.size();
         W.ntcol = (int32_t)tcol.size();
-        W.ntcolb = (int32_t)tcolb.size();
         W.ntgh = (int32_t)tgh.size();
         W.ntlk = (int32_t)tlk.size();
     }
@@ -848,18 +839,13 @@ hipError_t engine_op(lb_engine* e, int d, int64_t j) {
     const bool fill = (j & 1) == 0;
     if (W.ngh && fill) ETRY(k->ghost_fill(e->las, st, W.gh, W.ngh, j, e->storage, 0, e->stream));
     if (W.ncol)
-        ETRY(k->collide(e->las, st, W.col, W.ncol, j, e->storage, W.wide, 0, e->sched, e->waves, e->stream));
-    if (W.ncolb)
-        ETRY(k->collide(e->las, st, W.colb, W.ncolb, j, e->storage, W.wide, 1, e->sched, e->waves,
-                        e->stream));
+        ETRY(k->collide(e->las, st, W.col, W.ncol, j, e->storage, W.wide, e->sched, e->waves, e->stream));
     if (W.nlk) ETRY(k->bouzidi(e->las, st, W.lk, W.nlk, j, e->storage, 0, e->stream));
-    if (W.ntcol || W.ntcolb) {
+    if (W.ntcol) {
         // the thermal kernel has no persistent form
         const int tsched = e->sched == LB_SCHED_PERSISTENT ? LB_SCHED_LINEAR : e->sched;
         if (W.ntgh && fill) ETRY(k->ghost_fill(e->las, st, W.tgh, W.ntgh, j, e->storage, 1, e->stream));
-        if (W.ntcol) ETRY(k->thermal(e->las, st, W.tcol, W.ntcol, j, e->storage, W.wide_g, 0, tsched, e->stream));
-        if (W.ntcolb)
-            ETRY(k->thermal(e->las, st, W.tcolb, W.ntcolb, j, e->storage, W.wide_g, 1, tsched, e->stream));
+        ETRY(k->thermal(e->las, st, W.tcol, W.ntcol, j, e->storage, W.wide_g, tsched, e->stream));
         if (W.ntlk) ETRY(k->bouzidi(e->las, st, W.tlk, W.ntlk, j, e->storage, 1, e->stream));
     }
     if (d < e->lmax) {
@@ -1323,7 +1309,8 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
         L.order_host = order;
         std::vector<lbk::Work> wcol((size_t)nb);
         for (int32_t i = 0; i < nb; i++)
-            wcol[(size_t)i] = mkwork(L.id - 1, order[(size_t)i], 0, L.nbr + (size_t)order[(size_t)i] * Q);
+            wcol[(size_t)i] = mkwork(L.id - 1, order[(size_t)i], 0, L.nbr + (size_t)order[(size_t)i] * Q,
+                                     i < L.n_int ? 0 : lbk::WORK_BOUNDARY);
         RC(dalloc(c, &L.wcol, wcol.size()));
         RC(h2d(c, L.wcol, wcol.data(), wcol.size()));
         RC(h2d(c, L.obst, d->obstacle, n4));

@@ -115,9 +115,11 @@ struct Work {
     int32_t li;              // LevelArgs index
     int32_t item;            // block (stream-collide) or first entry of a 256-entry chunk
     int32_t ci;              // CaseState index
-    int32_t pad;
+    int32_t flags;           // stream-collide: WORK_* of the block
     const int32_t* nbr_row;  // the block's neighbour row (stream-collide), else null
 };
+// some neighbour of the block is neither a block nor a ghost block (domain boundary)
+constexpr int32_t WORK_BOUNDARY = 8;
 
 struct ForceArgs {
     // finest level
@@ -182,11 +184,10 @@ struct FiniteEntry {
 #define LBK_DECLARE(NS)                                                                                  \
     namespace NS {                                                                                       \
     hipError_t collide(const lbk::LevelArgs* las, const lbk::CaseState* states, const lbk::Work* work,    \
-                       int32_t n_tiles, int64_t j, int storage, int wide, int boundary, int sched,       \
-                       int waves, hipStream_t s);                                                        \
-    hipError_t thermal(const lbk::LevelArgs* las, const lbk::CaseState* states, const lbk::Work* work,    \
-                       int32_t n_tiles, int64_t j, int storage, int wide, int boundary, int sched,       \
+                       int32_t n_tiles, int64_t j, int storage, int wide, int sched, int waves,          \
                        hipStream_t s);                                                                   \
+    hipError_t thermal(const lbk::LevelArgs* las, const lbk::CaseState* states, const lbk::Work* work,    \
+                       int32_t n_tiles, int64_t j, int storage, int wide, int sched, hipStream_t s);     \
     hipError_t ghost_fill(const lbk::LevelArgs* las, const lbk::CaseState* states, const lbk::Work* work, int32_t n_chunks, int64_t j,  \
                           int storage, int thermal, hipStream_t s);                                      \
     hipError_t bouzidi(const lbk::LevelArgs* las, const lbk::CaseState* states, const lbk::Work* work, int32_t n_chunks, int64_t j,     \

@@ -7,8 +7,8 @@
 // goes through that block's neighbour-table row, staged in LDS; the centre
 // entry of the row is the block itself, so in-block and cross-block pulls are
 // one load instruction with a per-lane block index.  Sources with no
-// neighbour block fall to the boundary cascade (inlet/outlet equilibrium,
-// y/z mirror, coarse-to-fine interpolation), a non-inlined cold path.
+// neighbour block (domain boundary) take the boundary cascade
+// (inlet/outlet equilibrium, y/z mirror) in pull_mirrors.
 //
 // Operation order follows the reference kernels statement by statement (see
 // the citations), so that with -ffp-contract=off the results equal a plain
@@ -111,15 +111,17 @@ struct GhostArgs {
     int32_t temporal, comp, thermal;
 };
 
-// The case record, read through the global address space (uniform loads).
+// The case record, read through the global address space (uniform loads, in
+// 64-bit words: a 64-bit field assembled from two 32-bit ones comes back as a
+// vector load that every wave waits for before its first pull).
 __device__ __forceinline__ CaseState case_state(const CaseState* st) {
-    static_assert(sizeof(CaseState) % 4 == 0, "CaseState is read as 32-bit words");
-    typedef const __attribute__((address_space(1))) uint32_t GW;
+    static_assert(sizeof(CaseState) % 8 == 0, "CaseState is read as 64-bit words");
+    typedef const __attribute__((address_space(1))) uint64_t GW;
     const GW* src = (const GW*)st;
     CaseState out;
-    uint32_t* dst = reinterpret_cast<uint32_t*>(&out);
+    uint64_t* dst = reinterpret_cast<uint64_t*>(&out);
 #pragma unroll
-    for (unsigned i = 0; i < sizeof(CaseState) / 4; i++) dst[i] = src[i];
+    for (unsigned i = 0; i < sizeof(CaseState) / 8; i++) dst[i] = src[i];
     return out;
 }
 
@@ -256,6 +258,9 @@ typedef __attribute__((address_space(1))) uint8_t GU8;
 __device__ __forceinline__ const GF* gp(const float* p) { return (const GF*)p; }
 __device__ __forceinline__ GF* gp(float* p) { return (GF*)p; }
 __device__ __forceinline__ const GU8* gp(const uint8_t* p) { return (const GU8*)p; }
+__device__ __forceinline__ const __attribute__((address_space(1))) int32_t* gp(const int32_t* p) {
+    return (const __attribute__((address_space(1))) int32_t*)p;
+}
 typedef __attribute__((address_space(1))) uint16_t GU16;
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) v4u GV4U;
@@ -271,10 +276,13 @@ struct Codec<0> {
     static __device__ __forceinline__ float load(const void* base, size_t i, float) {
         return ((const GF*)base)[i];
     }
+    // stored bits at a byte offset, and their value
+    typedef float Raw;
     template <class OffT>
-    static __device__ __forceinline__ float loadb(const void* base, OffT off, float) {
+    static __device__ __forceinline__ Raw raw(const void* base, OffT off) {
         return *(const GF*)((const GC*)base + off);
     }
+    static __device__ __forceinline__ float value(Raw v, float) { return v; }
     static __device__ __forceinline__ void store(void* base, size_t i, float f, float) { ((GF*)base)[i] = f; }
     // non-temporal store, for the stream-collide outputs (read again only
     // one substep later, after the whole level has streamed through L2)
@@ -290,11 +298,12 @@ struct Codec<1> {
         const uint16_t u = ((const GU16*)base)[i];
         return w + __half2float(__ushort_as_half(u));
     }
+    typedef uint16_t Raw;
     template <class OffT>
-    static __device__ __forceinline__ float loadb(const void* base, OffT off, float w) {
-        const uint16_t u = *(const GU16*)((const GC*)base + off);
-        return w + __half2float(__ushort_as_half(u));
+    static __device__ __forceinline__ Raw raw(const void* base, OffT off) {
+        return *(const GU16*)((const GC*)base + off);
     }
+    static __device__ __forceinline__ float value(Raw u, float w) { return w + __half2float(__ushort_as_half(u)); }
     static __device__ __forceinline__ void store(void* base, size_t i, float f, float w) {
         ((GU16*)base)[i] = __half_as_ushort(__float2half_rn(f - w));
     }
@@ -311,11 +320,12 @@ struct Codec<2> {
         const uint32_t u = ((const GU16*)base)[i];
         return w + __uint_as_float(u << 16);
     }
+    typedef uint16_t Raw;
     template <class OffT>
-    static __device__ __forceinline__ float loadb(const void* base, OffT off, float w) {
-        const uint32_t u = *(const GU16*)((const GC*)base + off);
-        return w + __uint_as_float(u << 16);
+    static __device__ __forceinline__ Raw raw(const void* base, OffT off) {
+        return *(const GU16*)((const GC*)base + off);
     }
+    static __device__ __forceinline__ float value(Raw u, float w) { return w + __uint_as_float((uint32_t)u << 16); }
     static __device__ __forceinline__ uint16_t enc(float x) {
         uint32_t b = __float_as_uint(x);
         if ((b & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((b >> 16) | 0x40u);   // quiet NaN
@@ -411,25 +421,83 @@ __device__ __forceinline__ float wk_rt(int k) {
 }
 
 // Missing-neighbour cascade of stream_collide_cumulant! (kernel_cumulant.jl:117-159)
-// for sources outside the domain.  An in-domain source without a block (the
-// coarse-to-fine case of :143-156) never reaches here: it is a ghost block
-// filled by ghost_kernel.  The last branch (a level-1 source inside the
-// domain with no block) cannot occur either, level 1 being the full box; it
-// returns w_k as the reference does.
-template <int ST>
-__device__ __forceinline__ float bc_value(const CollideArgs& a, int k, int b, int c, int sgx, int sgy, int sgz, int gy,
-                                          int gz) {
-    float cx = (float)CX(k), cy = (float)CY(k), cz = (float)CZ(k), w = wk_rt(k);
-    if (sgx < 1) {
-        float noise = a.inlet_turb > 0.0f ? gradient_noise(gy, gz, a.seed, 1234) * a.inlet_turb * a.u_inlet : 0.0f;
-        float u_inst = a.u_inlet + noise;
-        return feq_auto(1.0f, u_inst, 0.0f, 0.0f, w, cx, cy, cz, a.comp);
+// for a pull whose source lies in no block of the level: x outside the domain
+// takes the inlet or outlet equilibrium, y (then z) outside mirrors the
+// direction at the cell's own slot, and a source inside the domain gives w_k
+// (an in-domain source of a refined level is a ghost block, never missing; on
+// level 1 it cannot occur with the full box).  Per axis and lattice component
+// + 1, whether the lane's source coordinate lies outside the domain.
+struct DomainSide {
+    bool xlo[3], xhi[3], y[3], z[3];
+};
+struct CellPos {
+    int x, y, z;  // 1-based global cell coordinates
+};
+__device__ __forceinline__ CellPos cell_pos(const int32_t* borg, int b, int c) {
+    const auto* o = gp(borg) + (size_t)b * 3;
+    return {o[0] + (c & 7) + 1, o[1] + ((c >> 3) & 7) + 1, o[2] + (c >> 6) + 1};
+}
+__device__ __forceinline__ DomainSide domain_side(const CellPos& p, int nxg, int nyg, int nzg) {
+    DomainSide s;
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const int sx = p.x - (i - 1), sy = p.y - (i - 1), sz = p.z - (i - 1);
+        s.xlo[i] = sx < 1;
+        s.xhi[i] = sx > nxg;
+        s.y[i] = sy < 1 || sy > nyg;
+        s.z[i] = sz < 1 || sz > nzg;
     }
-    if (sgx > a.nxg) return feq_auto(1.0f, a.u_inlet, 0.0f, 0.0f, w, cx, cy, cz, a.comp);
-    // the mirrored direction has the same |c|, hence the same weight
-    if (sgy < 1 || sgy > a.nyg) return Codec<ST>::load(a.f_in, fidx(b, MIRY(k), c), w);
-    if (sgz < 1 || sgz > a.nzg) return Codec<ST>::load(a.f_in, fidx(b, MIRZ(k), c), w);
-    return w;
+    return s;
+}
+
+// The pull of a cell: the 27 loads of its sources, all issued before any is
+// used, each one pull-table read (tab: the wave's 27 entries) and one add.  The
+// stored bits are decoded by the caller after its next barrier, so that no
+// wait on them comes before it.
+template <int ST>
+using Pulled = typename Codec<ST>::Raw;
+template <int ST, class OffT>
+__device__ __forceinline__ OffT pull_offset(const OffT* tab, int k, OffT cb, int e) {
+    constexpr int ESZ = ST == 0 ? 4 : 2;
+    return tab[e] + cb + (OffT)((512 * k - (CX(k) + 8 * CY(k) + 64 * CZ(k))) * ESZ);
+}
+// Table entry of direction k for a lane whose pulls in +x, -x, +y, -y leave
+// the block on the sides oxp, oxm, oyp, oym.
+__device__ __forceinline__ int pull_entry(int k, int oxp, int oxm, int oyp, int oym) {
+    const int ox = CX(k) == 1 ? oxp : (CX(k) == -1 ? oxm : 0);
+    const int oy = CY(k) == 1 ? oyp : (CY(k) == -1 ? oym : 0);
+    return 9 * (CZ(k) + 1) + (ox + 1) + 3 * (oy + 1);
+}
+template <int ST, class OffT>
+__device__ __forceinline__ void pull(const void* f, const OffT* tab, OffT cb, int oxp, int oxm, int oyp, int oym,
+                                     Pulled<ST> (&P)[27]) {
+#pragma unroll
+    for (int k = 0; k < 27; k++)
+        P[k] = Codec<ST>::raw(f, pull_offset<ST, OffT>(tab, k, cb, pull_entry(k, oxp, oxm, oyp, oym)));
+}
+// Boundary blocks: the missing sources that the mirror walls replace, loaded
+// from the cell's own slots in one round of loads behind the pull's (its own
+// loads of these directions read a harmless slot).  Returns the directions
+// whose source no slot holds, for the caller to fill in.  m: the wave's
+// missing-entry mask; own: byte offset of the cell's slot 0.
+template <int ST, class OffT>
+__device__ __forceinline__ uint32_t pull_mirrors(const void* f, uint32_t m, OffT own, int oxp, int oxm, int oyp,
+                                                 int oym, const DomainSide& ds, Pulled<ST> (&P)[27]) {
+    constexpr int ESZ = ST == 0 ? 4 : 2;
+    uint32_t empty = 0u;
+#pragma unroll
+    for (int k = 0; k < 27; k++) {
+        const uint32_t miss = (m >> pull_entry(k, oxp, oxm, oyp, oym)) & 1u;
+        const bool in_x = !ds.xlo[CX(k) + 1] && !ds.xhi[CX(k) + 1];
+        const bool my = ds.y[CY(k) + 1], mz = ds.z[CZ(k) + 1];
+        if (miss) {
+            if (in_x && (my || mz))
+                P[k] = Codec<ST>::raw(f, own + (my ? (OffT)(512 * MIRY(k) * ESZ) : (OffT)(512 * MIRZ(k) * ESZ)));
+            else
+                empty |= 1u << k;
+        }
+    }
+    return empty;
 }
 
 __device__ __forceinline__ void chim_fwd(float& fm, float& f0, float& fp, float u) {
@@ -494,7 +562,7 @@ __device__ __forceinline__ void build_pull_table(const int32_t* __restrict__ row
         const int ox = j % 3 - 1, oy = j / 3 - 1;
         const int zw = half * 4 + w;
         const int oz = (cz == 1 && zw == 0) ? -1 : ((cz == -1 && zw == 7) ? 1 : 0);
-        const int nbb = row[j + 9 * (oz + 1)];
+        const int nbb = gp(row)[j + 9 * (oz + 1)];
         const OffT bs = (OffT)(Q * NC);
         OffT v;
         if (nbb >= 0) {
@@ -540,7 +608,7 @@ __device__ __forceinline__ void build_vel_table(const int32_t* __restrict__ row,
             const int zw = half * 4 + w;
             const bool zedge = (dz == 1 && zw == 7) || (dz == -1 && zw == 0);
             if (dz == 0 || zedge) {
-                const int nbb = row[(dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)];
+                const int nbb = gp(row)[(dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)];
                 if (nbb >= 0 && nbb < nb)
                     v = (OffT)nbb * (OffT)(3 * NC * 4) - (OffT)(4 * (8 * dx + 64 * dy + 512 * dz));
                 else
@@ -617,56 +685,59 @@ __device__ __forceinline__ void vel_tile_store(const VelTile& t, int c, float* v
 // Occupancy: the collision needs ~160 VGPRs, which allows 3 waves per SIMD.
 // Capping the kernel's VGPRs (W waves per SIMD) spills values to scratch,
 // which stays in cache, and lets more waves hide the pull's memory latency.
-// Boundary blocks (some neighbour outside the domain) need the 27 KB cascade
-// buffer in LDS, which limits them to 5 work-groups per CU; they run at 5.
-// Interior blocks need no cascade buffer (their LDS holds the output tile and,
-// in FP32, the velocity tile: 14-23 KB); W = 5 or 6 is a launch option
-// (picked by the autotuner).  The two compile to the same floating-point
-// operations (tested bit-identical); a 4-wave build contracts differently and
-// is not offered.  Measured on the 52.5M-cell cube case with the staged
-// stores: 5 waves is best (6 waves spills more: FP32 +5 %, FP16 +7 %).
+// W = 5 or 6 is a launch option (picked by the autotuner); the two compile to
+// the same floating-point operations (tested bit-identical); a 4-wave build
+// contracts differently and is not offered.
+// Boundary blocks (some neighbour outside the domain, flagged in the work
+// entry) run in the same launch, as a second instance of the body behind one
+// uniform branch: a launch of their own is bound by latency (13-22 us for 24 to
+// 1,100 work-groups on the small cases, most of it the cascade's loads one
+// after the other), and nothing ran beside it.  With the mirrored sources
+// loaded in one round and no launch of its own, a coarse step went 63 -> 41 us
+// (55 k cells, 2 levels), 381 -> 338 us (1.3 M cells, 3 levels, FP32) and
+// 1.74 -> 1.65 ms (4.5 M cells, thermal); 2.09 -> 2.04 ms at 6.1 M cells.  The
+// two instances are kept apart because one body with the fix-up inside made
+// the 16-bit interior path a third slower (the populations' registers become
+// one tuple that is copied).
 //
 // collide_tile is one half-block tile (work-list entry wk, half `half`);
 // collide_kernel runs one tile per work-group, collide_kernel_persistent
 // (LB_SCHED_PERSISTENT) runs a grid of as many work-groups as fit the
 // device at once, each looping over the tiles in order.
+template <int ST>
+constexpr int OUT_ROWS = ST == 0 ? 14 : 27;  // rows of the collide's output tile
+
+// The tile's LDS: pull and stencil tables, output tile, velocity tile.  The
+// outputs leave through stream_tile.  The work-group's previous velocity with
+// its face halos goes through LDS for the WALE stencil (vel_tile_load /
+// _store), and in FP32 the output tile is halved so that both fit 5
+// work-groups per CU.  The velocity tile's loads are issued before the pull
+// and stored after it, so its barrier overlaps the pull's loads.  Measured on
+// the 52.5M-cell cube case, finest collide: FP32 -1.9 %, FP16 -3.1 % (with the
+// tile loads issued after the pull, FP16 lost 1.5 % to the barrier).
+template <int ST, class OffT>
+struct CollideLds {
+    __attribute__((aligned(16))) Stored<ST> out[4 * OUT_ROWS<ST> * 64];
+    float vt[3 * VT_SIZE];
+    OffT ptab[108];
+    OffT vtab[32];
+    uint64_t smask[2];
+};
+
 template <int ST, class OffT, bool BND>
-__device__ __forceinline__ void collide_tile(const LevelArgs* __restrict__ las, const CaseState* __restrict__ states,
-                                             const Work& wk, int half, int64_t j, int tid) {
-    __shared__ OffT ptab[108];
-    __shared__ OffT vtab[32];
-    __shared__ uint64_t smask[2];
-    __shared__ float sfix[BND ? 27 * 256 : 1];
-    // interior blocks: outputs leave through stream_tile (the boundary
-    // kernel's cascade buffer already takes the LDS budget)
-    constexpr bool STAGE = !BND;
-    // Interior blocks: the work-group's previous velocity with its face halos
-    // goes through LDS for the WALE stencil (vel_tile_load / _store), and in
-    // FP32 the output tile is halved so that both fit 5 work-groups per CU.
-    // The tile's loads are issued before the pull and stored after it, so
-    // its barrier overlaps the pull's loads.  Measured on the 52.5M-cell cube
-    // case, finest collide: FP32 -1.9 %, FP16 -3.1 % (with the tile loads
-    // issued after the pull, FP16 lost 1.5 % to the barrier).
-    constexpr bool VTILE = STAGE;
-    constexpr int ROWS = ST == 0 ? 14 : 27;
-    __shared__ __attribute__((aligned(16))) Stored<ST> sst[STAGE ? 4 * ROWS * 64 : 8];
-    __shared__ float vt[VTILE ? 3 * VT_SIZE : 1];
-    const LevelArgs& L = las[wk.li];
-    const int b = wk.item;
+__device__ __forceinline__ void collide_body(const CollideArgs& a, CollideLds<ST, OffT>& lds, int b, int half,
+                                             int tid) {
     constexpr int ESZ = ST == 0 ? 4 : 2;
+    constexpr int ROWS = OUT_ROWS<ST>;
+    // opaque to the boundary instance, so that nothing the two instances share
+    // is hoisted above the branch between them and kept live across it
+    if constexpr (BND) asm volatile("" : "+v"(tid));
     const int c = (half << 8) | tid;
-    // the neighbour-row loads go out together with the case record's
-    build_pull_table<OffT>(wk.nbr_row, b, half, (OffT)ESZ, ptab, smask, tid);
-    build_vel_table<OffT>(wk.nbr_row, L.nb, b, half, vtab, tid);
-    const CaseState S = case_state(states + wk.ci);
-    __syncthreads();
-    if (!live(L, S, j)) return;
-    const CollideArgs a = collide_view(L, S, j);
-    const int x = c & 7, y = (c >> 3) & 7, z = c >> 6;
+    const OffT* const ptab = lds.ptab;
+    const OffT* const vtab = lds.vtab;
+    float* const vt = lds.vt;
+    const int x = c & 7, y = (c >> 3) & 7;
     const int wv = tid >> 6;
-    const int gx = a.borg[b * 3 + 0] + x + 1;
-    const int gy = a.borg[b * 3 + 1] + y + 1;
-    const int gz = a.borg[b * 3 + 2] + z + 1;
     const size_t i4 = (size_t)b * NC + c;
     bool is_obs = false;
     if constexpr (ST != 0) is_obs = __builtin_nontemporal_load(&gp(a.obst)[i4]) != 0;
@@ -676,47 +747,21 @@ __device__ __forceinline__ void collide_tile(const LevelArgs* __restrict__ las, 
     const int oxp = x == 0 ? -1 : 0, oxm = x == 7 ? 1 : 0;
     const int oyp = y == 0 ? -1 : 0, oym = y == 7 ? 1 : 0;
     const OffT cb = (OffT)c * (OffT)ESZ;
-    VelTile vtl;
-    if constexpr (VTILE) vtl = vel_tile_load<OffT>(a.vel_in, vtab, half, c, tid);
-    float A[27];
-#pragma unroll
-    for (int k = 0; k < 27; k++) {
-        const int cx = CX(k), cy = CY(k), cz = CZ(k);
-        const int ox = cx == 1 ? oxp : (cx == -1 ? oxm : 0);
-        const int oy = cy == 1 ? oyp : (cy == -1 ? oym : 0);
-        const OffT off = ptab[wv * 27 + 9 * (cz + 1) + (ox + 1) + 3 * (oy + 1)] + cb +
-                         (OffT)((512 * k - (cx + 8 * cy + 64 * cz)) * ESZ);
-        A[k] = Codec<ST>::loadb(a.f_in, off, WK(k));
-    }
+    const VelTile vtl = vel_tile_load<OffT>(a.vel_in, vtab, half, c, tid);
+    Pulled<ST> P[27];
+    pull<ST, OffT>(a.f_in, ptab + wv * 27, cb, oxp, oxm, oyp, oym, P);
     // WALE stencil of the previous velocity, loaded together with the populations.
     float VN[6][3];
-    if constexpr (VTILE) {
-        vel_tile_store(vtl, c, vt, tid);
-        __syncthreads();
+    vel_tile_store(vtl, c, vt, tid);
+    __syncthreads();
 #pragma unroll
-        for (int n = 0; n < 6; n++) {
-            const int dx = n == 0 ? 1 : (n == 1 ? -1 : 0);
-            const int dy = n == 2 ? 1 : (n == 3 ? -1 : 0);
-            const int dz = n == 4 ? 1 : (n == 5 ? -1 : 0);
+    for (int n = 0; n < 6; n++) {
+        const int dx = n == 0 ? 1 : (n == 1 ? -1 : 0);
+        const int dy = n == 2 ? 1 : (n == 3 ? -1 : 0);
+        const int dz = n == 4 ? 1 : (n == 5 ? -1 : 0);
 #pragma unroll
-            for (int d = 0; d < 3; d++) VN[n][d] = vt[vt_index(d, wv + dz, y + dy, x + dx)];
-        }
-    } else {
-        const OffT own = vtab[wv * 8 + 6];
-#pragma unroll
-        for (int n = 0; n < 6; n++) {
-            const int dx = n == 0 ? 1 : (n == 1 ? -1 : 0);
-            const int dy = n == 2 ? 1 : (n == 3 ? -1 : 0);
-            const int dz = n == 4 ? 1 : (n == 5 ? -1 : 0);
-            const bool edge = n == 0 ? x == 7 : n == 1 ? x == 0 : n == 2 ? y == 7 : n == 3 ? y == 0 : true;
-            const OffT off = (edge ? vtab[wv * 8 + n] : own) + (OffT)(4 * (c + dx + 8 * dy + 64 * dz));
-            const GF* p = gaddr(a.vel_in, off);
-            VN[n][0] = p[0];
-            VN[n][1] = p[NC];
-            VN[n][2] = p[2 * NC];
-        }
+        for (int d = 0; d < 3; d++) VN[n][d] = vt[vt_index(d, wv + dz, y + dy, x + dx)];
     }
-    // lanes whose pull crosses into a missing block (domain boundary)
     // single-use inputs: non-temporal loads keep L2 for the neighbour pulls
     // FP32: a block with no solid, sponge or near-wall cell skips those loads
     // (the values they would give: not solid, sponge 0, no wall model); the
@@ -726,36 +771,32 @@ __device__ __forceinline__ void collide_tile(const LevelArgs* __restrict__ las, 
     // 2.3 % to the extra branch and keep the unconditional loads (bfl = 7).
     uint32_t bfl = 7u;
     if constexpr (ST == 0) {
-        bfl = a.bflags[b];
+        bfl = gp(a.bflags)[b];
         is_obs = (bfl & 4u) ? __builtin_nontemporal_load(&gp(a.obst)[i4]) != 0 : false;
     }
     const float sp = (bfl & 1u) ? __builtin_nontemporal_load(&gp(a.sponge)[i4]) : 0.0f;
     const float wdist =
         (a.wall_model == 1 && (bfl & 2u)) ? __builtin_nontemporal_load(&gp(a.wall_dist)[i4]) : 0.0f;
-    if constexpr (BND) {
-        uint32_t miss = 0u;
-        const uint32_t m = wave_miss(smask, wv);
-        if (m != 0u) {
+    uint32_t empty = 0u;
+    if constexpr (BND)
+        empty = pull_mirrors<ST, OffT>(a.f_in, wave_miss(lds.smask, wv), (OffT)b * (OffT)(Q * NC * ESZ) + cb, oxp, oxm,
+                                       oyp, oym, domain_side(cell_pos(a.borg, b, c), a.nxg, a.nyg, a.nzg), P);
+    float A[27];
 #pragma unroll
-            for (int k = 0; k < 27; k++) {
-                const int cx = CX(k), cy = CY(k), cz = CZ(k);
-                const int ox = cx == 1 ? oxp : (cx == -1 ? oxm : 0);
-                const int oy = cy == 1 ? oyp : (cy == -1 ? oym : 0);
-                miss |= ((m >> (9 * (cz + 1) + (ox + 1) + 3 * (oy + 1))) & 1u) << k;
-            }
-        }
-        // Boundary cascade for sources in no block: one inlined copy of the
-        // cascade in a rolled loop over k, results passed through LDS (a
-        // register array cannot be indexed by a run-time k without spilling).
-        if (miss != 0u) {
-#pragma unroll 1
-            for (int k = 0; k < 27; k++)
-                if (miss & (1u << k))
-                    sfix[k * 256 + tid] =
-                        bc_value<ST>(a, k, b, c, gx - CX(k), gy - CY(k), gz - CZ(k), gy, gz);
+    for (int k = 0; k < 27; k++) A[k] = Codec<ST>::value(P[k], WK(k));
+    if (BND && empty != 0u) {
+        const CellPos p = cell_pos(a.borg, b, c);
+        const float noise =
+            a.inlet_turb > 0.0f ? gradient_noise(p.y, p.z, a.seed, 1234) * a.inlet_turb * a.u_inlet : 0.0f;
+        const float u_inst = a.u_inlet + noise;
 #pragma unroll
-            for (int k = 0; k < 27; k++)
-                if (miss & (1u << k)) A[k] = sfix[k * 256 + tid];
+        for (int k = 0; k < 27; k++) {
+            if (!(empty & (1u << k))) continue;
+            const bool lo = p.x - CX(k) < 1, hi = p.x - CX(k) > a.nxg;
+            // uy = uz = 0: the equilibrium depends on c_x and |c| alone
+            const float v =
+                feq_auto(1.0f, lo ? u_inst : a.u_inlet, 0.0f, 0.0f, 1.0f, (float)CX(k), 0.0f, 0.0f, a.comp);
+            A[k] = lo || hi ? WK(k) * v : WK(k);
         }
     }
     float rho = 0.0f, jx = 0.0f, jy = 0.0f, jz = 0.0f;
@@ -782,20 +823,14 @@ __device__ __forceinline__ void collide_tile(const LevelArgs* __restrict__ las, 
         vo[iv + NC] = 0.0f;
         vo[iv + 2 * NC] = 0.0f;
         if (a.store_rho) ro[i4] = 1.0f;
-        if constexpr (STAGE) {
 #pragma unroll
-            for (int k = 0; k < 13; k++) {
-                const float t = A[k];
-                A[k] = A[OPP(k)];
-                A[OPP(k)] = t;
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < 27; k++) Codec<ST>::stream(fo, fidx(b, k, c), A[OPP(k)], WK(k));
-            return;
+        for (int k = 0; k < 13; k++) {
+            const float t = A[k];
+            A[k] = A[OPP(k)];
+            A[OPP(k)] = t;
         }
     }
-    // (staged form: solid cells skip the collision and join the store)
+    // (solid cells skip the collision and join the store)
     if (!is_obs) {
 
         // STEP 2: macroscopic + sponge + wall model (kernel_cumulant.jl:190-259)
@@ -1065,36 +1100,48 @@ __device__ __forceinline__ void collide_tile(const LevelArgs* __restrict__ las, 
                 float ft = WK(k) * 3.0f *
                            ((cxf - ux + 3.0f * cu * cxf) * Fx + (cyf - uy + 3.0f * cu * cyf) * Fy +
                             (czf - uz + 3.0f * cu * czf) * Fz);
-                if constexpr (STAGE)
-                    A[k] = A[k] + pre * ft;
-                else
-                    Codec<ST>::stream(fo, fidx(b, k, c), A[k] + pre * ft, WK(k));
+                A[k] = A[k] + pre * ft;
             }
-        } else if constexpr (!STAGE) {
-#pragma unroll
-            for (int k = 0; k < 27; k++) Codec<ST>::stream(fo, fidx(b, k, c), A[k], WK(k));
         }
     }  // !is_obs
-    if constexpr (STAGE) stream_tile<ST, ROWS>(fo, b, c, A, sst + wv * (ROWS * 64));
+    stream_tile<ST, ROWS>(fo, b, c, A, lds.out + wv * (ROWS * 64));
 }
 
-template <int ST, class OffT, bool BND, int W>
+template <int ST, class OffT>
+__device__ __forceinline__ void collide_tile(const LevelArgs* __restrict__ las, const CaseState* __restrict__ states,
+                                             const Work& wk, int half, int64_t j, int tid) {
+    __shared__ CollideLds<ST, OffT> lds;
+    const LevelArgs& L = las[wk.li];
+    const int b = wk.item;
+    // the neighbour-row loads go out together with the case record's
+    build_pull_table<OffT>(wk.nbr_row, b, half, (OffT)(ST == 0 ? 4 : 2), lds.ptab, lds.smask, tid);
+    build_vel_table<OffT>(wk.nbr_row, L.nb, b, half, lds.vtab, tid);
+    const CaseState S = case_state(states + wk.ci);
+    __syncthreads();
+    if (!live(L, S, j)) return;
+    const CollideArgs a = collide_view(L, S, j);
+    if (wk.flags & WORK_BOUNDARY)
+        collide_body<ST, OffT, true>(a, lds, b, half, tid);
+    else
+        collide_body<ST, OffT, false>(a, lds, b, half, tid);
+}
+
+template <int ST, class OffT, int W>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(W, W)))
 collide_kernel(const LevelArgs* __restrict__ las, const CaseState* __restrict__ states,
                const Work* __restrict__ work, int32_t n_tiles, int64_t j, int32_t sched) {
     Work wk;
     int half;
     if (!schedule(work, n_tiles, sched, wk, half)) return;
-    collide_tile<ST, OffT, BND>(las, states, wk, half, j, (int)threadIdx.x);
+    collide_tile<ST, OffT>(las, states, wk, half, j, (int)threadIdx.x);
 }
 
 // Persistent form: work-group g takes tiles g, g + G, g + 2G, ... in order.
 // All waves of a work-group make the same passes, and a barrier ends each
 // pass, so the LDS tables of a tile are not rewritten while any wave still
-// reads them.  A tile's early exits are uniform over the work-group (a case
-// past its last step) or come after the tile's last barrier (a solid lane's
-// bounce-back in the boundary form), so every wave reaches every barrier.
-template <int ST, class OffT, bool BND>
+// reads them.  A tile's early exit (a case past its last step) is uniform over
+// the work-group, so every wave reaches every barrier.
+template <int ST, class OffT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 5)))
 collide_kernel_persistent(const LevelArgs* __restrict__ las, const CaseState* __restrict__ states,
                           const Work* __restrict__ work, int32_t n_tiles, int64_t j) {
@@ -1105,7 +1152,7 @@ collide_kernel_persistent(const LevelArgs* __restrict__ las, const CaseState* __
         // the loop and kept live across the whole tile.
         int tid = (int)threadIdx.x;
         asm volatile("" : "+v"(tid));
-        collide_tile<ST, OffT, BND>(las, states, wk, (int)(logical & 1u), j, tid);
+        collide_tile<ST, OffT>(las, states, wk, (int)(logical & 1u), j, tid);
         __syncthreads();
     }
 }
@@ -1130,122 +1177,80 @@ inline unsigned persistent_groups(int n_tiles) {
 
 template <int ST, class OffT>
 void collide_launch(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_tiles, int64_t j,
-                    int boundary, int sched, int waves, hipStream_t s) {
+                    int sched, int waves, hipStream_t s) {
     const dim3 t(256);
     if (sched == LB_SCHED_PERSISTENT) {
         const dim3 g(persistent_groups(n_tiles));
-        if (boundary)
-            hipLaunchKernelGGL((collide_kernel_persistent<ST, OffT, true>), g, t, 0, s, las, states, work, n_tiles, j);
-        else
-            hipLaunchKernelGGL((collide_kernel_persistent<ST, OffT, false>), g, t, 0, s, las, states, work, n_tiles, j);
+        hipLaunchKernelGGL((collide_kernel_persistent<ST, OffT>), g, t, 0, s, las, states, work, n_tiles, j);
         return;
     }
     const dim3 g(padded_groups(n_tiles));
-    if (boundary)
-        hipLaunchKernelGGL((collide_kernel<ST, OffT, true, 5>), g, t, 0, s, las, states, work, n_tiles, j, sched);
-    else if (waves == 6)
-        hipLaunchKernelGGL((collide_kernel<ST, OffT, false, 6>), g, t, 0, s, las, states, work, n_tiles, j, sched);
+    if (waves == 6)
+        hipLaunchKernelGGL((collide_kernel<ST, OffT, 6>), g, t, 0, s, las, states, work, n_tiles, j, sched);
     else
-        hipLaunchKernelGGL((collide_kernel<ST, OffT, false, 5>), g, t, 0, s, las, states, work, n_tiles, j, sched);
+        hipLaunchKernelGGL((collide_kernel<ST, OffT, 5>), g, t, 0, s, las, states, work, n_tiles, j, sched);
 }
 
-// boundary = 0 requires every block of the work list to have all 26
-// neighbours (blocks or ghost blocks).  waves: occupancy of the interior
-// kernel (5 or 6 waves per SIMD).
+// Work entries whose block has a missing neighbour (ghost blocks count as
+// present) carry WORK_BOUNDARY.  waves: occupancy (5 or 6 waves per SIMD).
 hipError_t collide(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_tiles, int64_t j,
-                   int storage, int wide, int boundary, int sched, int waves, hipStream_t s) {
+                   int storage, int wide, int sched, int waves, hipStream_t s) {
     if (n_tiles <= 0) return hipSuccess;
     if (wide) {
-        if (storage == 1) collide_launch<1, uint64_t>(las, states, work, n_tiles, j, boundary, sched, waves, s);
-        else if (storage == 2) collide_launch<2, uint64_t>(las, states, work, n_tiles, j, boundary, sched, waves, s);
-        else collide_launch<0, uint64_t>(las, states, work, n_tiles, j, boundary, sched, waves, s);
+        if (storage == 1) collide_launch<1, uint64_t>(las, states, work, n_tiles, j, sched, waves, s);
+        else if (storage == 2) collide_launch<2, uint64_t>(las, states, work, n_tiles, j, sched, waves, s);
+        else collide_launch<0, uint64_t>(las, states, work, n_tiles, j, sched, waves, s);
     } else {
-        if (storage == 1) collide_launch<1, uint32_t>(las, states, work, n_tiles, j, boundary, sched, waves, s);
-        else if (storage == 2) collide_launch<2, uint32_t>(las, states, work, n_tiles, j, boundary, sched, waves, s);
-        else collide_launch<0, uint32_t>(las, states, work, n_tiles, j, boundary, sched, waves, s);
+        if (storage == 1) collide_launch<1, uint32_t>(las, states, work, n_tiles, j, sched, waves, s);
+        else if (storage == 2) collide_launch<2, uint32_t>(las, states, work, n_tiles, j, sched, waves, s);
+        else collide_launch<0, uint32_t>(las, states, work, n_tiles, j, sched, waves, s);
     }
     return hipGetLastError();
 }
 
 // ---------------------------------------------------------------------------
 // Thermal DDF (src/collision/kernel_thermal.jl:14-202)
-template <int ST>
-__device__ __forceinline__ float thermal_bc(const ThermalArgs& a, int k, int b, int c, int sgx, int sgy, int sgz) {
-    float cx = (float)CX(k), cy = (float)CY(k), cz = (float)CZ(k), w = wk_rt(k);
-    if (sgx < 1) return geq(a.T_inlet, a.u_inlet, 0.0f, 0.0f, w, cx, cy, cz);
-    if (sgx > a.nxg) return geq(a.T_inlet, a.u_inlet, 0.0f, 0.0f, w, cx, cy, cz);
-    if (sgy < 1 || sgy > a.nyg) return Codec<ST>::load(a.g_in, fidx(b, MIRY(k), c), w);
-    if (sgz < 1 || sgz > a.nzg) return Codec<ST>::load(a.g_in, fidx(b, MIRZ(k), c), w);
-    // in-domain sources without a block are ghost blocks (thermal ghost fill)
-    return w * a.T_inlet;
-}
+template <int ST, class OffT>
+struct ThermalLds {
+    __attribute__((aligned(16))) Stored<ST> out[4 * 27 * 64];  // outputs leave through stream_tile, as in the collide
+    OffT ptab[108];
+    uint64_t smask[2];
+};
 
 template <int ST, class OffT, bool BND>
-__global__ void __launch_bounds__(256) thermal_kernel(const LevelArgs* __restrict__ las,
-                                                      const CaseState* __restrict__ states,
-                                                      const Work* __restrict__ work, int32_t n_tiles, int64_t j,
-                                                      int32_t sched) {
-    __shared__ OffT ptab[108];
-    __shared__ uint64_t smask[2];
-    __shared__ float sfix[BND ? 27 * 256 : 1];
-    // interior blocks: outputs leave through stream_tile, as in the collide
-    constexpr bool STAGE = !BND;
-    __shared__ __attribute__((aligned(16))) Stored<ST> sst[STAGE ? 4 * 27 * 64 : 8];
-    Work wk;
-    int half;
-    if (!schedule(work, n_tiles, sched, wk, half)) return;
-    const LevelArgs& L = las[wk.li];
-    const int b = wk.item;
-    const int c = (half << 8) | threadIdx.x;
+__device__ __forceinline__ void thermal_body(const ThermalArgs& a, ThermalLds<ST, OffT>& lds, int b, int half,
+                                             int tid) {
     constexpr int ESZ = ST == 0 ? 4 : 2;
-    build_pull_table<OffT>(wk.nbr_row, b, half, (OffT)ESZ, ptab, smask, (int)threadIdx.x);
-    const CaseState S = case_state(states + wk.ci);
-    __syncthreads();
-    if (!live(L, S, j)) return;
-    const ThermalArgs a = thermal_view(L, S, j);
-    const int x = c & 7, y = (c >> 3) & 7, z = c >> 6;
-    const int wv = threadIdx.x >> 6;
-    const int gx = a.borg[b * 3 + 0] + x + 1;
-    const int gy = a.borg[b * 3 + 1] + y + 1;
-    const int gz = a.borg[b * 3 + 2] + z + 1;
+    if constexpr (BND) asm volatile("" : "+v"(tid));  // as in collide_body
+    const int c = (half << 8) | tid;
+    const OffT* const ptab = lds.ptab;
+    const int x = c & 7, y = (c >> 3) & 7;
+    const int wv = tid >> 6;
     const size_t i4 = (size_t)b * NC + c;
     const size_t iv = (size_t)b * 3 * NC + c;
     float ux = gp(a.vel)[iv], uy = gp(a.vel)[iv + NC], uz = gp(a.vel)[iv + 2 * NC];
     const int oxp = x == 0 ? -1 : 0, oxm = x == 7 ? 1 : 0;
     const int oyp = y == 0 ? -1 : 0, oym = y == 7 ? 1 : 0;
     const OffT cb = (OffT)c * (OffT)ESZ;
+    Pulled<ST> P[27];
+    pull<ST, OffT>(a.g_in, ptab + wv * 27, cb, oxp, oxm, oyp, oym, P);
+    const bool is_obs = gp(a.obst)[i4] != 0;
+    uint32_t empty = 0u;
+    if constexpr (BND)
+        empty = pull_mirrors<ST, OffT>(a.g_in, wave_miss(lds.smask, wv), (OffT)b * (OffT)(Q * NC * ESZ) + cb, oxp, oxm,
+                                       oyp, oym, domain_side(cell_pos(a.borg, b, c), a.nxg, a.nyg, a.nzg), P);
     float G[27];
 #pragma unroll
-    for (int k = 0; k < 27; k++) {
-        const int cx = CX(k), cy = CY(k), cz = CZ(k);
-        const int ox = cx == 1 ? oxp : (cx == -1 ? oxm : 0);
-        const int oy = cy == 1 ? oyp : (cy == -1 ? oym : 0);
-        const OffT off = ptab[wv * 27 + 9 * (cz + 1) + (ox + 1) + 3 * (oy + 1)] + cb +
-                         (OffT)((512 * k - (cx + 8 * cy + 64 * cz)) * ESZ);
-        G[k] = Codec<ST>::loadb(a.g_in, off, WK(k));
-    }
-    const bool is_obs = gp(a.obst)[i4] != 0;
-    if constexpr (BND) {
-        // boundary blocks only: sources in no block take the boundary cascade
-        uint32_t miss = 0u;
-        const uint32_t m = wave_miss(smask, wv);
-        if (m != 0u) {
+    for (int k = 0; k < 27; k++) G[k] = Codec<ST>::value(P[k], WK(k));
+    if (BND && empty != 0u) {
+        // inlet and outlet equilibria at the inlet temperature
+        const CellPos p = cell_pos(a.borg, b, c);
 #pragma unroll
-            for (int k = 0; k < 27; k++) {
-                const int cx = CX(k), cy = CY(k), cz = CZ(k);
-                const int ox = cx == 1 ? oxp : (cx == -1 ? oxm : 0);
-                const int oy = cy == 1 ? oyp : (cy == -1 ? oym : 0);
-                miss |= ((m >> (9 * (cz + 1) + (ox + 1) + 3 * (oy + 1))) & 1u) << k;
-            }
-        }
-        if (miss != 0u) {
-#pragma unroll 1
-            for (int k = 0; k < 27; k++)
-                if (miss & (1u << k))
-                    sfix[k * 256 + threadIdx.x] = thermal_bc<ST>(a, k, b, c, gx - CX(k), gy - CY(k), gz - CZ(k));
-#pragma unroll
-            for (int k = 0; k < 27; k++)
-                if (miss & (1u << k)) G[k] = sfix[k * 256 + threadIdx.x];
+        for (int k = 0; k < 27; k++) {
+            if (!(empty & (1u << k))) continue;
+            const bool out = p.x - CX(k) < 1 || p.x - CX(k) > a.nxg;
+            G[k] = out ? geq(a.T_inlet, a.u_inlet, 0.0f, 0.0f, WK(k), (float)CX(k), (float)CY(k), (float)CZ(k))
+                       : WK(k) * a.T_inlet;
         }
     }
     float Tsum = 0.0f;
@@ -1262,13 +1267,9 @@ __global__ void __launch_bounds__(256) thermal_kernel(const LevelArgs* __restric
                 float gw = geq(a.T_wall, 0.0f, 0.0f, 0.0f, WK(k), (float)CX(k), (float)CY(k), (float)CZ(k));
                 go = 2.0f * gw - gopp;
             }
-            if constexpr (STAGE)
-                G[k] = go;
-            else
-                Codec<ST>::stream(a.g_out, fidx(b, k, c), go, WK(k));
+            G[k] = go;
         }
         if (a.store_T) a.T_out[i4] = a.adiabatic == 1 ? Tsum : a.T_wall;
-        if constexpr (!STAGE) return;
     } else {
         float Tl = fmaxf(Tsum, 0.01f);
         const float sp = a.sponge[i4];
@@ -1288,37 +1289,45 @@ __global__ void __launch_bounds__(256) thermal_kernel(const LevelArgs* __restric
                 gs = gs * (1.0f - sp) + gt * sp;
             }
             float ge = geq(Tl, ux, uy, uz, WK(k), (float)CX(k), (float)CY(k), (float)CZ(k));
-            if constexpr (STAGE)
-                G[k] = gs - omg * (gs - ge);
-            else
-                Codec<ST>::stream(a.g_out, fidx(b, k, c), gs - omg * (gs - ge), WK(k));
+            G[k] = gs - omg * (gs - ge);
         }
     }  // !is_obs
-    if constexpr (STAGE) stream_tile<ST, 27>(a.g_out, b, c, G, sst + wv * (27 * 64));
+    stream_tile<ST, 27>(a.g_out, b, c, G, lds.out + wv * (27 * 64));
 }
 
-// Interior blocks (every neighbour present, ghosts included) run the variant
-// without the boundary cascade and its 27 KiB LDS buffer, which would limit
-// occupancy to 5 work-groups per CU.
 template <int ST, class OffT>
-void thermal_launch2(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_tiles, int64_t j,
-                     int boundary, int sched, hipStream_t s) {
-    const dim3 g(padded_groups(n_tiles)), t(256);
-    if (boundary) hipLaunchKernelGGL((thermal_kernel<ST, OffT, true>), g, t, 0, s, las, states, work, n_tiles, j, sched);
-    else hipLaunchKernelGGL((thermal_kernel<ST, OffT, false>), g, t, 0, s, las, states, work, n_tiles, j, sched);
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ST == 0 ? 5 : 7)))
+thermal_kernel(const LevelArgs* __restrict__ las, const CaseState* __restrict__ states,
+               const Work* __restrict__ work, int32_t n_tiles, int64_t j, int32_t sched) {
+    __shared__ ThermalLds<ST, OffT> lds;
+    Work wk;
+    int half;
+    if (!schedule(work, n_tiles, sched, wk, half)) return;
+    const LevelArgs& L = las[wk.li];
+    build_pull_table<OffT>(wk.nbr_row, wk.item, half, (OffT)(ST == 0 ? 4 : 2), lds.ptab, lds.smask, (int)threadIdx.x);
+    const CaseState S = case_state(states + wk.ci);
+    __syncthreads();
+    if (!live(L, S, j)) return;
+    const ThermalArgs a = thermal_view(L, S, j);
+    if (wk.flags & WORK_BOUNDARY)
+        thermal_body<ST, OffT, true>(a, lds, wk.item, half, (int)threadIdx.x);
+    else
+        thermal_body<ST, OffT, false>(a, lds, wk.item, half, (int)threadIdx.x);
 }
+
 template <int ST>
 void thermal_launch(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_tiles, int64_t j,
-                    int wide, int boundary, int sched, hipStream_t s) {
-    if (wide) thermal_launch2<ST, uint64_t>(las, states, work, n_tiles, j, boundary, sched, s);
-    else thermal_launch2<ST, uint32_t>(las, states, work, n_tiles, j, boundary, sched, s);
+                    int wide, int sched, hipStream_t s) {
+    const dim3 g(padded_groups(n_tiles)), t(256);
+    if (wide) hipLaunchKernelGGL((thermal_kernel<ST, uint64_t>), g, t, 0, s, las, states, work, n_tiles, j, sched);
+    else hipLaunchKernelGGL((thermal_kernel<ST, uint32_t>), g, t, 0, s, las, states, work, n_tiles, j, sched);
 }
 hipError_t thermal(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_tiles, int64_t j,
-                   int storage, int wide, int boundary, int sched, hipStream_t s) {
+                   int storage, int wide, int sched, hipStream_t s) {
     if (n_tiles <= 0) return hipSuccess;
-    if (storage == 1) thermal_launch<1>(las, states, work, n_tiles, j, wide, boundary, sched, s);
-    else if (storage == 2) thermal_launch<2>(las, states, work, n_tiles, j, wide, boundary, sched, s);
-    else thermal_launch<0>(las, states, work, n_tiles, j, wide, boundary, sched, s);
+    if (storage == 1) thermal_launch<1>(las, states, work, n_tiles, j, wide, sched, s);
+    else if (storage == 2) thermal_launch<2>(las, states, work, n_tiles, j, wide, sched, s);
+    else thermal_launch<0>(las, states, work, n_tiles, j, wide, sched, s);
     return hipGetLastError();
 }
 
