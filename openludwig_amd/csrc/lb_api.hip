@@ -13,7 +13,7 @@
 //     buffers in the reference, are ping-ponged by step parity so the previous
 //     step's values survive as rho_old / T_old.
 //   * f_post_collision is not allocated: Bouzidi gathers its inputs from the
-//     uncorrected f_out before scattering the corrected slots.
+//     uncorrected f_out before it stores the corrected slots.
 //   * No device synchronisation between launches; everything is ordered on
 //     the context's stream.
 #include <hip/hip_runtime.h>
@@ -46,7 +46,7 @@ struct Kern {
                           int, hipStream_t);
     hipError_t (*ghost_fill)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int, int,
                              hipStream_t);
-    hipError_t (*bouzidi)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int, int,
+    hipError_t (*bouzidi)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int,
                           hipStream_t);
     hipError_t (*set_state)(lbk::CaseState*, const lbk::CaseState&, hipStream_t);
     hipError_t (*advance)(lbk::CaseState*, int32_t, hipStream_t);
@@ -97,15 +97,12 @@ struct Level {
     std::vector<int32_t> grid_host;  // host copy of grid, for the child level's ghost parents
     // Bouzidi link list
     int64_t nlinks = 0;
-    // Bouzidi link slots: uint32 (lidx32, a population buffer below 2^32
-    // slots) or int64
-    void* ldst = nullptr;
-    void* ls1 = nullptr;
-    void* ls2 = nullptr;
+    // BouzidiLink<uint32_t> (lidx32, a population buffer below 2^32 slots) or
+    // <uint64_t>, and the work entries' (first link, number of links)
+    void* llink = nullptr;
     bool lidx32 = false;
-    float* la = nullptr;
-    float* lb = nullptr;
     float* ltmp = nullptr;
+    std::vector<std::pair<int32_t, int32_t>> lchunks;
     bool wide = false;    // population buffer >= 4 GiB: kernels use 64-bit offsets
     bool wide_g = false;  // the same for the thermal populations
     // work lists over this level alone (LevelArgs index = level index):
@@ -175,8 +172,8 @@ struct EngineCase {
 
 // Work lists of one depth of the engine's recursion (concatenated over cases).
 struct DepthWork {
-    lbk::Work *col = nullptr, *gh = nullptr, *lk = nullptr, *tcol = nullptr, *tgh = nullptr, *tlk = nullptr;
-    int32_t ncol = 0, ngh = 0, nlk = 0, ntcol = 0, ntgh = 0, ntlk = 0;
+    lbk::Work *col = nullptr, *gh = nullptr, *lk = nullptr, *tcol = nullptr, *tgh = nullptr;
+    int32_t ncol = 0, ngh = 0, nlk = 0, ntcol = 0, ntgh = 0;
     int wide = 0, wide_g = 0;
     // force sampling of the cases whose first level runs at this depth:
     // triangle chunks (li = record, item = chunk) and the record indices
@@ -431,52 +428,94 @@ int build_links(lb_ctx* c, Level& L, const lb_level_desc* d) {
     }
     L.nlinks = (int64_t)dst.size();
     if (L.nlinks == 0) return LB_OK;
-    size_t n = (size_t)L.nlinks;
-    // Link order does not change results (every link is gathered before any
-    // is scattered, and each destination slot has one link).  Sorted by
-    // destination, a wave's links share (block, direction) rows, so the
-    // scatter's stores and the gather's loads of the same row coalesce.
-    {
-        std::vector<size_t> perm(n);
-        for (size_t i = 0; i < n; i++) perm[i] = i;
-        std::sort(perm.begin(), perm.end(), [&](size_t u, size_t v) { return dst[u] < dst[v]; });
-        auto apply = [&](auto& vec) {
-            auto tmp = vec;
-            for (size_t i = 0; i < n; i++) vec[i] = tmp[perm[i]];
-        };
-        apply(dst);
-        apply(s1);
-        apply(s2);
-        apply(ca);
-        apply(cb);
+    const size_t n = (size_t)L.nlinks;
+    if (n > (size_t)INT32_MAX) return fail(c, LB_EINVAL, "level %d: %zu wall links", d->level_id, n);
+    // Link order.  Sorted by destination, a wave's links share (block,
+    // direction) rows, so its loads and stores of the same row coalesce.  A
+    // work entry gathers its links' values before it stores any, so a link that
+    // reads a slot which another link corrects (a cell with walls on both
+    // sides, or two cells apart from one) has to be in the same entry: linked
+    // links stand together, and entries of up to 256 links are cut between
+    // such groups (one longer group makes one longer entry).
+    std::vector<int32_t> by_dst(n), group(n);
+    for (size_t i = 0; i < n; i++) by_dst[i] = (int32_t)i;
+    std::sort(by_dst.begin(), by_dst.end(), [&](int32_t u, int32_t v) { return dst[(size_t)u] < dst[(size_t)v]; });
+    for (size_t r = 0; r < n; r++) group[r] = (int32_t)r;  // over ranks in by_dst; the root is the lowest rank
+    auto root = [&](int32_t r) {
+        while (group[(size_t)r] != r) r = group[(size_t)r] = group[(size_t)group[(size_t)r]];
+        return r;
+    };
+    // corrected slots as bits, per block that has any: few reads meet one
+    std::vector<int32_t> block_row((size_t)nb, -1);
+    std::vector<uint64_t> bits;
+    constexpr size_t kRow = (size_t)Q * NC / 64;
+    for (size_t i = 0; i < n; i++) {
+        const size_t blk = (size_t)dst[i] / (Q * NC), at = (size_t)dst[i] % (Q * NC);
+        if (block_row[blk] < 0) {
+            block_row[blk] = (int32_t)(bits.size() / kRow);
+            bits.resize(bits.size() + kRow, 0);
+        }
+        bits[(size_t)block_row[blk] * kRow + at / 64] |= 1ull << (at % 64);
     }
-    // 32-bit slot indices where the level's population buffer (ghost blocks
-    // and padding included) has fewer than 2^32 slots: 12 instead of 24 of
-    // the link's 40 bytes of data (gather and scatter read the link data on
-    // every substep).  wide_offsets keeps 64-bit indices too.
+    auto corrected = [&](int64_t slot) {
+        const size_t blk = (size_t)slot / (Q * NC), at = (size_t)slot % (Q * NC);
+        return block_row[blk] >= 0 && ((bits[(size_t)block_row[blk] * kRow + at / 64] >> (at % 64)) & 1u) != 0;
+    };
+    for (size_t r = 0; r < n; r++) {
+        const size_t i = (size_t)by_dst[r];
+        for (const int64_t slot : {s1[i], s2[i]}) {
+            if (slot == dst[i] || !corrected(slot)) continue;
+            const auto it = std::lower_bound(by_dst.begin(), by_dst.end(), slot,
+                                             [&](int32_t u, int64_t v) { return dst[(size_t)u] < v; });
+            if (it == by_dst.end() || dst[(size_t)*it] != slot) continue;
+            const int32_t a = root((int32_t)r), b = root((int32_t)(it - by_dst.begin()));
+            group[(size_t)std::max(a, b)] = std::min(a, b);
+        }
+    }
+    std::unordered_map<int32_t, std::vector<int32_t>> members;  // groups of more than one link
+    for (size_t r = 0; r < n; r++) {
+        const int32_t g = root((int32_t)r);
+        if (g != (int32_t)r) members[g].push_back((int32_t)r);
+    }
+    std::vector<int32_t> order;  // ranks, group by group
+    order.reserve(n);
+    L.lchunks.clear();
+    int32_t first = 0;
+    for (size_t r = 0; r < n; r++) {
+        if (group[r] != (int32_t)r) continue;  // listed with its group
+        const auto it = members.find((int32_t)r);
+        const int32_t size = 1 + (it == members.end() ? 0 : (int32_t)it->second.size());
+        const int32_t have = (int32_t)order.size() - first;
+        if (have > 0 && have + size > 256) {
+            L.lchunks.emplace_back(first, have);
+            first = (int32_t)order.size();
+        }
+        order.push_back((int32_t)r);
+        if (it != members.end()) order.insert(order.end(), it->second.begin(), it->second.end());
+    }
+    L.lchunks.emplace_back(first, (int32_t)order.size() - first);
+    // 32-bit slots where the level's population buffer (ghost blocks and
+    // padding included) has fewer than 2^32 of them.  wide_offsets keeps
+    // 64-bit slots too.
     const uint64_t slots = ((uint64_t)nb + (uint64_t)L.ngh) * NC * Q + 512;
     L.lidx32 = c->cfg.wide_offsets == 0 && slots < ((uint64_t)1 << 32);
-    auto upload_slots = [&](const std::vector<int64_t>& v, void** out) -> int {
-        if (L.lidx32) {
-            std::vector<uint32_t> v32(v.begin(), v.end());
-            uint32_t* p = nullptr;
-            RC(dalloc(c, &p, n));
-            *out = p;
-            return h2d(c, p, v32.data(), n);
+    auto upload_links = [&](auto zero) -> int {
+        typedef decltype(zero) SlotT;
+        std::vector<lbk::BouzidiLink<SlotT>> v(n);
+        for (size_t q = 0; q < n; q++) {
+            const size_t i = (size_t)by_dst[(size_t)order[q]];
+            v[q] = {(SlotT)dst[i], (SlotT)s2[i], ca[i], cb[i]};
         }
-        int64_t* p = nullptr;
+        lbk::BouzidiLink<SlotT>* p = nullptr;
         RC(dalloc(c, &p, n));
-        *out = p;
+        L.llink = p;
         return h2d(c, p, v.data(), n);
     };
-    RC(upload_slots(dst, &L.ldst));
-    RC(upload_slots(s1, &L.ls1));
-    RC(upload_slots(s2, &L.ls2));
-    RC(dalloc(c, &L.la, n));
-    RC(dalloc(c, &L.lb, n));
-    RC(dalloc(c, &L.ltmp, n));
-    RC(h2d(c, L.la, ca.data(), n));
-    RC(h2d(c, L.lb, cb.data(), n));
+    if (L.lidx32) RC(upload_links((uint32_t)0));
+    else RC(upload_links((uint64_t)0));
+    bool longer = false;
+    for (const auto& e : L.lchunks) longer = longer || e.second > 256;
+    if (longer) RC(dalloc(c, &L.ltmp, n));
     return LB_OK;
 }
 
@@ -525,15 +564,14 @@ int step_level(lb_ctx* c, int li, int64_t j) {
         HIPCHK(c, c->k->collide(las, st, L.wcol, L.nb, j, storage, L.wide ? 1 : 0, LB_SCHED_LINEAR,
                                 default_waves(storage), c->stream));
         if (e1) HIPCHK(c, hipEventRecord(e1, c->stream));
-        if (L.n_lchunks > 0) HIPCHK(c, c->k->bouzidi(las, st, L.wlk, L.n_lchunks, j, storage, 0, c->stream));
         if (ddf) {
             if (fill) HIPCHK(c, c->k->ghost_fill(las, st, L.wgh, L.n_gchunks, j, storage, 1, c->stream));
             hipEvent_t e2 = nullptr;
             RC(profile_begin(c, L, 1, &e2));
             HIPCHK(c, c->k->thermal(las, st, L.wcol, L.nb, j, storage, L.wide_g ? 1 : 0, LB_SCHED_LINEAR, c->stream));
             if (e2) HIPCHK(c, hipEventRecord(e2, c->stream));
-            if (L.n_lchunks > 0) HIPCHK(c, c->k->bouzidi(las, st, L.wlk, L.n_lchunks, j, storage, 1, c->stream));
         }
+        if (L.n_lchunks > 0) HIPCHK(c, c->k->bouzidi(las, st, L.wlk, L.n_lchunks, j, storage, c->stream));
     }
     RC(step_level(c, li + 1, 2 * j));
     RC(step_level(c, li + 1, 2 * j + 1));
@@ -590,7 +628,17 @@ int item_list(lb_ctx* c, int li, int32_t n, lbk::Work** out, int32_t* n_items) {
     return h2d(c, *out, w.data(), w.size());
 }
 
-// Work list of 256-item chunks of one level (ghost entries, Bouzidi links).
+// Work list of a level's wall links.
+int link_list(lb_ctx* c, int li, Level& L) {
+    L.n_lchunks = L.nlinks > 0 ? (int32_t)L.lchunks.size() : 0;
+    if (L.n_lchunks == 0) return LB_OK;
+    std::vector<lbk::Work> w;
+    for (const auto& e : L.lchunks) w.push_back(mkwork(li, e.first, 0, nullptr, e.second));
+    RC(dalloc(c, &L.wlk, w.size()));
+    return h2d(c, L.wlk, w.data(), w.size());
+}
+
+// Work list of 256-item chunks of one level (ghost entries).
 int chunk_list(lb_ctx* c, int li, int64_t n, lbk::Work** out, int32_t* n_chunks) {
     *n_chunks = (int32_t)((n + 255) / 256);
     if (*n_chunks == 0) return LB_OK;
@@ -651,11 +699,7 @@ int upload_level_args(lb_ctx* c, int li) {
     A.gbmask = L.gbmask;
     A.ngent = L.ngent;
     A.links.n = L.nlinks;
-    A.links.dst = L.ldst;
-    A.links.s1 = L.ls1;
-    A.links.s2 = L.ls2;
-    A.links.a = L.la;
-    A.links.b = L.lb;
+    A.links.link = L.llink;
     A.links.tmp = L.ltmp;
     A.links.idx32 = L.lidx32 ? 1 : 0;
     return h2d(c, c->las_dev + li, &A, 1);
@@ -770,7 +814,7 @@ int engine_rebuild(lb_engine* e) {
         W.nfrec = (int32_t)frec[(size_t)d - 1].size();
     }
     for (int d = 1; d <= e->lmax; d++) {
-        std::vector<lbk::Work> col, colb, gh, lk, tcol, tcolb, tgh, tlk;  // colb, tcolb: boundary blocks, listed last
+        std::vector<lbk::Work> col, colb, gh, lk, tcol, tcolb, tgh;  // colb, tcolb: boundary blocks, listed last
         DepthWork& W = e->depth[(size_t)d - 1];
         for (size_t i = 0; i < e->cases.size(); i++) {
             const lb_ctx* c = e->cases[i].c;
@@ -797,10 +841,7 @@ int engine_rebuild(lb_engine* e) {
                     gh.push_back(mkwork(li, item, ci, nullptr));
                     if (ddf) tgh.push_back(mkwork(li, item, ci, nullptr));
                 }
-            for (int64_t q = 0; q < lev.nlinks; q += 256) {
-                lk.push_back(mkwork(li, (int)q, ci, nullptr));
-                if (ddf) tlk.push_back(mkwork(li, (int)q, ci, nullptr));
-            }
+            for (const auto& ch : lev.lchunks) lk.push_back(mkwork(li, ch.first, ci, nullptr, ch.second));
             if (lev.wide) W.wide = 1;
             if (lev.wide_g) W.wide_g = 1;
         }
@@ -811,13 +852,11 @@ int engine_rebuild(lb_engine* e) {
         RC(eupload(e, &W.lk, lk));
         RC(eupload(e, &W.tcol, tcol));
         RC(eupload(e, &W.tgh, tgh));
-        RC(eupload(e, &W.tlk, tlk));
         W.ncol = (int32_t)col.size();
         W.ngh = (int32_t)gh.size();
         W.nlk = (int32_t)lk.size();
         W.ntcol = (int32_t)tcol.size();
         W.ntgh = (int32_t)tgh.size();
-        W.ntlk = (int32_t)tlk.size();
     }
     e->n_active = (int32_t)e->cases.size();
     e->dirty = false;
@@ -840,14 +879,13 @@ hipError_t engine_op(lb_engine* e, int d, int64_t j) {
     if (W.ngh && fill) ETRY(k->ghost_fill(e->las, st, W.gh, W.ngh, j, e->storage, 0, e->stream));
     if (W.ncol)
         ETRY(k->collide(e->las, st, W.col, W.ncol, j, e->storage, W.wide, e->sched, e->waves, e->stream));
-    if (W.nlk) ETRY(k->bouzidi(e->las, st, W.lk, W.nlk, j, e->storage, 0, e->stream));
     if (W.ntcol) {
         // the thermal kernel has no persistent form
         const int tsched = e->sched == LB_SCHED_PERSISTENT ? LB_SCHED_LINEAR : e->sched;
         if (W.ntgh && fill) ETRY(k->ghost_fill(e->las, st, W.tgh, W.ntgh, j, e->storage, 1, e->stream));
         ETRY(k->thermal(e->las, st, W.tcol, W.ntcol, j, e->storage, W.wide_g, tsched, e->stream));
-        if (W.ntlk) ETRY(k->bouzidi(e->las, st, W.tlk, W.ntlk, j, e->storage, 1, e->stream));
     }
+    if (W.nlk) ETRY(k->bouzidi(e->las, st, W.lk, W.nlk, j, e->storage, e->stream));
     if (d < e->lmax) {
         ETRY(engine_op(e, d + 1, 2 * j));
         ETRY(engine_op(e, d + 1, 2 * j + 1));
@@ -1342,7 +1380,7 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
     RC(build_links(c, L, d));
     if (staged) RC(item_list(c, L.id - 1, L.ngent > 0 ? ngh : 0, &L.wgh, &L.n_gchunks));
     else RC(chunk_list(c, L.id - 1, L.ngent, &L.wgh, &L.n_gchunks));
-    RC(chunk_list(c, L.id - 1, L.nlinks, &L.wlk, &L.n_lchunks));
+    RC(link_list(c, L.id - 1, L));
     RC(upload_level_args(c, L.id - 1));
     L.uploaded = true;
     return LB_OK;

@@ -46,16 +46,21 @@ struct CaseState {
     int32_t adiabatic, temporal;
 };
 
-// Bouzidi link list: corrected slot dst = a*f[s1] + b*f[s2], all indices
-// into one population buffer (block-major layout).  The slot indices are
-// uint32 when idx32 (a buffer below 2^32 slots), else int64.
+// Bouzidi link: corrected slot dst = a*f[s1] + b*f[s2], slots of one
+// population buffer (block-major layout).  s1 is the opposite direction at
+// dst's own cell (slot dst + (26 - 2k) 512 for dst's direction k).
+template <class SlotT>
+struct BouzidiLink {
+    SlotT dst, s2;
+    float a, b;
+};
+// The link list, uint32 slots when idx32 (a buffer below 2^32 slots), else
+// uint64.  Links that read a slot which another link corrects are listed in
+// one work entry with it (see build_links), so that a work-group may correct
+// in place after a barrier.  tmp: values of work entries over 256 links, or null.
 struct BouzidiLinks {
     int64_t n;
-    const void* dst;
-    const void* s1;
-    const void* s2;
-    const float* a;
-    const float* b;
+    const void* link;
     float* tmp;
     int32_t idx32;
     int32_t pad;
@@ -113,9 +118,9 @@ struct LevelArgs {
 // issued together.
 struct Work {
     int32_t li;              // LevelArgs index
-    int32_t item;            // block (stream-collide) or first entry of a 256-entry chunk
+    int32_t item;            // block (stream-collide), first entry of a chunk, or ghost block
     int32_t ci;              // CaseState index
-    int32_t flags;           // stream-collide: WORK_* of the block
+    int32_t flags;           // stream-collide: WORK_* of the block; links: entries of the chunk
     const int32_t* nbr_row;  // the block's neighbour row (stream-collide), else null
 };
 // some neighbour of the block is neither a block nor a ghost block (domain boundary)
@@ -191,7 +196,7 @@ struct FiniteEntry {
     hipError_t ghost_fill(const lbk::LevelArgs* las, const lbk::CaseState* states, const lbk::Work* work, int32_t n_chunks, int64_t j,  \
                           int storage, int thermal, hipStream_t s);                                      \
     hipError_t bouzidi(const lbk::LevelArgs* las, const lbk::CaseState* states, const lbk::Work* work, int32_t n_chunks, int64_t j,     \
-                       int storage, int thermal, hipStream_t s);                                         \
+                       int storage, hipStream_t s);                                                      \
     hipError_t set_state(lbk::CaseState* st, const lbk::CaseState& v, hipStream_t s);                   \
     hipError_t advance(lbk::CaseState* st, int32_t n, hipStream_t s);                             \
     hipError_t init_level(void* f0, void* f1, float* rho0, float* rho1, float* v0, float* v1, int32_t nb,  \

@@ -681,7 +681,7 @@ __device__ __forceinline__ void vel_tile_store(const VelTile& t, int c, float* v
 
 // stream_collide_cumulant! (src/collision/kernel_cumulant.jl:29-627), with the
 // A/B buffers chosen by the caller and no f_post_collision copy (Bouzidi
-// reads f_out before it corrects it, see bouzidi_gather below).
+// reads f_out before it corrects it, see bouzidi_kernel below).
 // Occupancy: the collision needs ~160 VGPRs, which allows 3 waves per SIMD.
 // Capping the kernel's VGPRs (W waves per SIMD) spills values to scratch,
 // which stays in cache, and lets more waves hide the pull's memory latency.
@@ -1749,74 +1749,104 @@ hipError_t ghost_fill(const LevelArgs* las, const CaseState* states, const Work*
 }
 
 // ---------------------------------------------------------------------------
-// Bouzidi (src/geometry/bouzidi_kernel.jl:13-92) as two sparse passes over
-// the link list: gather every corrected value from the uncorrected
-// post-collision populations, then scatter.  Each link's destination slot is
-// distinct, so the result equals the reference's read-from-f_post_collision
-// form without its full-size copy.  __fmul_rn/__fadd_rn keep the two
-// products and the sum rounded separately in both builds.
-// All three slots of a link have the same |c|, so one weight w_k (from the
-// destination's direction) decodes and encodes them.
-// The corrected buffer is the substep's output half (f_out, or g_out).
-__device__ __forceinline__ void* bouzidi_target(const LevelArgs& L, const CaseState& S, int64_t j, int thermal) {
-    const int out = 1 - (int)(substep(L, S, j) & 1);
-    return thermal ? (void*)L.g[out] : L.f[out];
+// Bouzidi (src/geometry/bouzidi_kernel.jl:13-92) as one sparse pass over the
+// link list: a work-group gathers the corrected values of its work entry from
+// the uncorrected post-collision populations, and after a barrier stores them.
+// Each link's destination slot is distinct, and a link that reads a slot which
+// another link corrects shares its work entry (build_links), so the result
+// equals the reference's read-from-f_post_collision form without its full-size
+// copy.  With the thermal form one launch corrects f and g (their links are the
+// same), so the link data is read once.  __fmul_rn/__fadd_rn keep the two
+// products and the sum rounded separately in both builds.  All three slots of
+// a link have the same |c|, so one weight w_k (from the destination's
+// direction) decodes and encodes them.
+// Bound by latency (a chain of work entry, records, link, populations; then the
+// launch itself): as a gather pass and a scatter pass with the values through
+// memory, f and g apart, it took 4.8 + 5.3 us of a substep on the 1.3 M-cell
+// sphere (15 k links; a coarse step of 4 such substeps went 338 -> 328 us) and
+// 2 x (18.2 + 9.6) us on the 10.7 M-cell thermal wing in 16-bit storage (2 M
+// links; coarse step 5.14 -> 4.86 ms).
+template <int ST>
+struct LinkValue {
+    size_t d;
+    float w, v;
+};
+template <int ST, class SlotT>
+__device__ __forceinline__ LinkValue<ST> link_gather(const void* f, const BouzidiLink<SlotT>& l) {
+    LinkValue<ST> r;
+    r.d = (size_t)l.dst;
+    const int k = (int)((uint32_t)(l.dst >> 9) % 27u);
+    r.w = wk_rt(k);
+    const float f1 = Codec<ST>::load(f, r.d + (size_t)(ptrdiff_t)((26 - 2 * k) * NC), r.w);
+    const float f2 = Codec<ST>::load(f, (size_t)l.s2, r.w);
+    r.v = __fadd_rn(__fmul_rn(l.a, f1), __fmul_rn(l.b, f2));
+    return r;
 }
-// Slot index i of a link array (uint32 or int64 entries, uniform per level).
-__device__ __forceinline__ size_t link_slot(const BouzidiLinks& l, const void* p, int64_t i) {
-    typedef const __attribute__((address_space(1))) uint32_t GU32;
-    typedef const __attribute__((address_space(1))) int64_t GI64;
-    return l.idx32 ? (size_t)((GU32*)p)[i] : (size_t)((GI64*)p)[i];
+template <int ST, class SlotT>
+__device__ __forceinline__ void bouzidi_chunk(const BouzidiLinks& ls, const Work& wk, void* f, void* g) {
+    typedef BouzidiLink<SlotT> Link;
+    typedef const __attribute__((address_space(1))) uint32_t GW;
+    auto link_at = [&](int64_t i) {
+        Link l;
+        const GW* p = (const GW*)((const Link*)ls.link + i);
+        uint32_t* q = reinterpret_cast<uint32_t*>(&l);
+#pragma unroll
+        for (unsigned m = 0; m < sizeof(Link) / 4; m++) q[m] = p[m];
+        return l;
+    };
+    const int tid = (int)threadIdx.x;
+    if (wk.flags <= 256) {
+        LinkValue<ST> a{}, b{};
+        if (tid < wk.flags) {
+            const Link l = link_at((int64_t)wk.item + tid);
+            a = link_gather<ST>(f, l);
+            if (g) b = link_gather<ST>(g, l);
+        }
+        __syncthreads();
+        if (tid < wk.flags) {
+            Codec<ST>::store(f, a.d, a.v, a.w);
+            if (g) Codec<ST>::store(g, b.d, b.v, b.w);
+        }
+        return;
+    }
+    // a longer entry (a chain of links through each other's slots): values
+    // through memory, each read back by the work-item that wrote it
+    for (int pass = 0; pass < (g ? 2 : 1); pass++) {
+        void* x = pass == 0 ? f : g;
+        for (int i = tid; i < wk.flags; i += 256) {
+            const int64_t at = (int64_t)wk.item + i;
+            ls.tmp[at] = link_gather<ST>(x, link_at(at)).v;
+        }
+        __syncthreads();
+        for (int i = tid; i < wk.flags; i += 256) {
+            const int64_t at = (int64_t)wk.item + i;
+            const size_t d = (size_t)link_at(at).dst;
+            Codec<ST>::store(x, d, ls.tmp[at], wk_rt((int)((uint32_t)(d >> 9) % 27u)));
+        }
+    }
 }
 template <int ST>
-__global__ void __launch_bounds__(256) bouzidi_gather(const LevelArgs* __restrict__ las,
+__global__ void __launch_bounds__(256) bouzidi_kernel(const LevelArgs* __restrict__ las,
                                                       const CaseState* __restrict__ states,
-                                                      const Work* __restrict__ work, int64_t j, int thermal) {
+                                                      const Work* __restrict__ work, int64_t j) {
     const Work wk = work[blockIdx.x];
     const LevelArgs& L = las[wk.li];
     const CaseState S = case_state(states + wk.ci);
     if (!live(L, S, j)) return;
-    const BouzidiLinks& l = L.links;
-    const int64_t i = (int64_t)wk.item + threadIdx.x;
-    if (i >= l.n) return;
-    const void* f = bouzidi_target(L, S, j, thermal);
-    const float w = wk_rt((int)((link_slot(l, l.dst, i) >> 9) % 27));
-    const float f1 = Codec<ST>::load(f, link_slot(l, l.s1, i), w), f2 = Codec<ST>::load(f, link_slot(l, l.s2, i), w);
-    l.tmp[i] = __fadd_rn(__fmul_rn(l.a[i], f1), __fmul_rn(l.b[i], f2));
-}
-template <int ST>
-__global__ void __launch_bounds__(256) bouzidi_scatter(const LevelArgs* __restrict__ las,
-                                                       const CaseState* __restrict__ states,
-                                                       const Work* __restrict__ work, int64_t j, int thermal) {
-    const Work wk = work[blockIdx.x];
-    const LevelArgs& L = las[wk.li];
-    const CaseState S = case_state(states + wk.ci);
-    if (!live(L, S, j)) return;
-    const BouzidiLinks& l = L.links;
-    const int64_t i = (int64_t)wk.item + threadIdx.x;
-    if (i >= l.n) return;
-    void* f = bouzidi_target(L, S, j, thermal);
-    const size_t d = link_slot(l, l.dst, i);
-    const float w = wk_rt((int)((d >> 9) % 27));
-    Codec<ST>::store(f, d, l.tmp[i], w);
+    const int out = 1 - (int)(substep(L, S, j) & 1);  // the substep's output half
+    if (L.links.idx32) bouzidi_chunk<ST, uint32_t>(L.links, wk, L.f[out], L.g[out]);
+    else bouzidi_chunk<ST, uint64_t>(L.links, wk, L.f[out], L.g[out]);
 }
 
-template <int ST>
-void bouzidi_launch(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_chunks, int64_t j,
-                    int thermal, hipStream_t s) {
-    const dim3 g((unsigned)n_chunks), t(256);
-    hipLaunchKernelGGL(bouzidi_gather<ST>, g, t, 0, s, las, states, work, j, thermal);
-    hipLaunchKernelGGL(bouzidi_scatter<ST>, g, t, 0, s, las, states, work, j, thermal);
-}
-
-// One work-group per work entry (LevelArgs index, first of 256 links).
-hipError_t bouzidi(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_chunks, int64_t j, int storage, int thermal,
-                   hipStream_t s) {
+// One work-group per work entry (LevelArgs index, first link, number of
+// links); corrects f, and g where the level has it.
+hipError_t bouzidi(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_chunks, int64_t j,
+                   int storage, hipStream_t s) {
     if (n_chunks <= 0) return hipSuccess;
-    const int st = storage;
-    if (st == 1) bouzidi_launch<1>(las, states, work, n_chunks, j, thermal, s);
-    else if (st == 2) bouzidi_launch<2>(las, states, work, n_chunks, j, thermal, s);
-    else bouzidi_launch<0>(las, states, work, n_chunks, j, thermal, s);
+    const dim3 g((unsigned)n_chunks), t(256);
+    if (storage == 1) hipLaunchKernelGGL(bouzidi_kernel<1>, g, t, 0, s, las, states, work, j);
+    else if (storage == 2) hipLaunchKernelGGL(bouzidi_kernel<2>, g, t, 0, s, las, states, work, j);
+    else hipLaunchKernelGGL(bouzidi_kernel<0>, g, t, 0, s, las, states, work, j);
     return hipGetLastError();
 }
 
