@@ -273,6 +273,13 @@ int h2d(lb_ctx* c, T* dst, const T* src, size_t n) {
     return LB_OK;
 }
 
+// Brings what was allocated since `before` up to `bytes`.
+int keep_bytes(lb_ctx* c, int64_t before, int64_t bytes) {
+    const int64_t missing = before + bytes - c->bytes;
+    uint8_t* p = nullptr;
+    return missing > 0 ? dalloc(c, &p, (size_t)missing) : LB_OK;
+}
+
 float half_to_float(uint16_t h) {
     int s = (h >> 15) & 1, e = (h >> 10) & 31, m = h & 1023;
     float v;
@@ -1377,10 +1384,16 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
         RC(h2d(c, L.grid, grid.data(), ng));
         L.grid_host = std::move(grid);
     }
+    const int64_t before_links = c->bytes;
     RC(build_links(c, L, d));
+    RC(link_list(c, L.id - 1, L));
+    // A case's footprint is a number that hosts plan with and keep (admission
+    // budgets, recorded sizes), so tables that got smaller leave it as it is:
+    // the links' 6 arrays (3 slots, 2 weights, 1 value) and chunks of 256.
+    RC(keep_bytes(c, before_links,
+                  L.nlinks * (3 * (L.lidx32 ? 4 : 8) + 12) + (L.nlinks + 255) / 256 * (int64_t)sizeof(lbk::Work)));
     if (staged) RC(item_list(c, L.id - 1, L.ngent > 0 ? ngh : 0, &L.wgh, &L.n_gchunks));
     else RC(chunk_list(c, L.id - 1, L.ngent, &L.wgh, &L.n_gchunks));
-    RC(link_list(c, L.id - 1, L));
     RC(upload_level_args(c, L.id - 1));
     L.uploaded = true;
     return LB_OK;

@@ -111,6 +111,7 @@ struct LevelArgs {
     const uint32_t* gbmask;
     int64_t ngent;
     BouzidiLinks links;
+    int64_t reserved[4];  // the record's size is part of a case's footprint
 };
 
 // Work list entry.  The neighbour row travels with the entry so that the
