@@ -1851,7 +1851,7 @@ hipError_t bouzidi(const LevelArgs* las, const CaseState* states, const Work* wo
 }
 
 // Case state updates.  set_state writes a whole record (single-case stepping,
-// once per coarse step); advance moves every case of an engine by its
+// once per lb_step_batch call); advance moves every case of an engine by its
 // step increment and looks up the inlet velocity of the new ramp batch.
 __global__ void set_state_kernel(CaseState* st, const CaseState v) {
     if (threadIdx.x == 0) *st = v;
