@@ -44,7 +44,7 @@ struct Kern {
                           int, int, hipStream_t);
     hipError_t (*thermal)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int, int,
                           int, hipStream_t);
-    hipError_t (*ghost_fill)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int, int,
+    hipError_t (*ghost_fill)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int,
                              hipStream_t);
     hipError_t (*bouzidi)(const lbk::LevelArgs*, const lbk::CaseState*, const lbk::Work*, int32_t, int64_t, int,
                           hipStream_t);
@@ -87,12 +87,10 @@ struct Level {
     int32_t* grid = nullptr;
     // ghost blocks (coarse-to-fine interface sources)
     int32_t ngh = 0;
-    int64_t ngent = 0;
-    int32_t* gent = nullptr;
-    int32_t* gpar = nullptr;     // FP32: per ghost entry, its 8 parent cells, (block << 9) | cell, or -1
-    int32_t* gstart = nullptr;   // 16-bit: per ghost block, its first entry (ngh + 1 values)
-    int32_t* gregion = nullptr;  // 16-bit: per ghost block, its 125 parent cells, (block << 9) | cell, or -1
-    uint32_t* gbmask = nullptr;  // 16-bit: per ghost block, the directions any of its entries serves
+    int32_t* gpb = nullptr;       // per ghost block: the 8 parent blocks around it, or -1
+    uint32_t* ggroup = nullptr;   // group and pair words of the chunks (lb_kernels.h)
+    uint32_t* gpair = nullptr;
+    lbk::GhostChunk* gchunk = nullptr;
     int32_t pd[3] = {0, 0, 0};
     std::vector<int32_t> grid_host;  // host copy of grid, for the child level's ghost parents
     // Bouzidi link list
@@ -106,9 +104,9 @@ struct Level {
     bool wide = false;    // population buffer >= 4 GiB: kernels use 64-bit offsets
     bool wide_g = false;  // the same for the thermal populations
     // work lists over this level alone (LevelArgs index = level index):
-    // blocks in processing order, ghost-entry chunks, Bouzidi-link chunks
+    // blocks in processing order, ghost-fill chunks, Bouzidi-link chunks
     lbk::Work* wcol = nullptr;
-    int32_t n_gchunks = 0;  // ghost fill work items: 256-entry chunks (FP32) or ghost blocks (16-bit)
+    int32_t n_gchunks = 0;
     lbk::Work* wgh = nullptr;
     int32_t n_lchunks = 0;
     lbk::Work* wlk = nullptr;
@@ -172,8 +170,8 @@ struct EngineCase {
 
 // Work lists of one depth of the engine's recursion (concatenated over cases).
 struct DepthWork {
-    lbk::Work *col = nullptr, *gh = nullptr, *lk = nullptr, *tcol = nullptr, *tgh = nullptr;
-    int32_t ncol = 0, ngh = 0, nlk = 0, ntcol = 0, ntgh = 0;
+    lbk::Work *col = nullptr, *gh = nullptr, *lk = nullptr, *tcol = nullptr;
+    int32_t ncol = 0, ngh = 0, nlk = 0, ntcol = 0;
     int wide = 0, wide_g = 0;
     // force sampling of the cases whose first level runs at this depth:
     // triangle chunks (li = record, item = chunk) and the record indices
@@ -565,14 +563,13 @@ int step_level(lb_ctx* c, int li, int64_t j) {
     if (L.nb > 0) {
         // one ghost pass per parent step fills the inputs of both child substeps
         const bool fill = li > 0 && L.n_gchunks > 0 && (j & 1) == 0;
-        if (fill) HIPCHK(c, c->k->ghost_fill(las, st, L.wgh, L.n_gchunks, j, storage, 0, c->stream));
+        if (fill) HIPCHK(c, c->k->ghost_fill(las, st, L.wgh, L.n_gchunks, j, storage, c->stream));
         hipEvent_t e1 = nullptr;
         RC(profile_begin(c, L, 0, &e1));
         HIPCHK(c, c->k->collide(las, st, L.wcol, L.nb, j, storage, L.wide ? 1 : 0, LB_SCHED_LINEAR,
                                 default_waves(storage), c->stream));
         if (e1) HIPCHK(c, hipEventRecord(e1, c->stream));
         if (ddf) {
-            if (fill) HIPCHK(c, c->k->ghost_fill(las, st, L.wgh, L.n_gchunks, j, storage, 1, c->stream));
             hipEvent_t e2 = nullptr;
             RC(profile_begin(c, L, 1, &e2));
             HIPCHK(c, c->k->thermal(las, st, L.wcol, L.nb, j, storage, L.wide_g ? 1 : 0, LB_SCHED_LINEAR, c->stream));
@@ -625,16 +622,6 @@ void set_current(lb_ctx* c, int64_t t) {
     }
 }
 
-// Work list of items 0 .. n - 1 of one level (ghost blocks).
-int item_list(lb_ctx* c, int li, int32_t n, lbk::Work** out, int32_t* n_items) {
-    *n_items = n;
-    if (n == 0) return LB_OK;
-    std::vector<lbk::Work> w((size_t)n);
-    for (int32_t i = 0; i < n; i++) w[(size_t)i] = mkwork(li, i, 0, nullptr);
-    RC(dalloc(c, out, w.size()));
-    return h2d(c, *out, w.data(), w.size());
-}
-
 // Work list of a level's wall links.
 int link_list(lb_ctx* c, int li, Level& L) {
     L.n_lchunks = L.nlinks > 0 ? (int32_t)L.lchunks.size() : 0;
@@ -645,14 +632,13 @@ int link_list(lb_ctx* c, int li, Level& L) {
     return h2d(c, L.wlk, w.data(), w.size());
 }
 
-// Work list of 256-item chunks of one level (ghost entries).
-int chunk_list(lb_ctx* c, int li, int64_t n, lbk::Work** out, int32_t* n_chunks) {
-    *n_chunks = (int32_t)((n + 255) / 256);
-    if (*n_chunks == 0) return LB_OK;
-    std::vector<lbk::Work> w((size_t)*n_chunks);
-    for (int32_t i = 0; i < *n_chunks; i++) w[(size_t)i] = mkwork(li, i * 256, 0, nullptr);
-    RC(dalloc(c, out, w.size()));
-    return h2d(c, *out, w.data(), w.size());
+// Work list of a level's ghost-fill chunks.
+int ghost_list(lb_ctx* c, int li, Level& L) {
+    if (L.n_gchunks == 0) return LB_OK;
+    std::vector<lbk::Work> w((size_t)L.n_gchunks);
+    for (int32_t i = 0; i < L.n_gchunks; i++) w[(size_t)i] = mkwork(li, i, 0, (const int32_t*)(L.gchunk + i));
+    RC(dalloc(c, &L.wgh, w.size()));
+    return h2d(c, L.wgh, w.data(), w.size());
 }
 
 // LevelArgs of level li (host copy + device record); the parent's pairs come
@@ -692,19 +678,12 @@ int upload_level_args(lb_ctx* c, int li) {
             A.pg[i] = P.g[i];
             A.pT[i] = P.T[i];
         }
-        A.pgrid = P.grid;
-        A.pdx = P.pd[0];
-        A.pdy = P.pd[1];
-        A.pdz = P.pd[2];
         A.ptau = P.tau;
         A.ptau_g = P.tau_g;
     }
-    A.gent = L.gent;
-    A.gpar = L.gpar;
-    A.gstart = L.gstart;
-    A.gregion = L.gregion;
-    A.gbmask = L.gbmask;
-    A.ngent = L.ngent;
+    A.gpb = L.gpb;
+    A.ggroup = L.ggroup;
+    A.gpair = L.gpair;
     A.links.n = L.nlinks;
     A.links.link = L.llink;
     A.links.tmp = L.ltmp;
@@ -821,7 +800,7 @@ int engine_rebuild(lb_engine* e) {
         W.nfrec = (int32_t)frec[(size_t)d - 1].size();
     }
     for (int d = 1; d <= e->lmax; d++) {
-        std::vector<lbk::Work> col, colb, gh, lk, tcol, tcolb, tgh;  // colb, tcolb: boundary blocks, listed last
+        std::vector<lbk::Work> col, colb, gh, lk, tcol, tcolb;  // colb, tcolb: boundary blocks, listed last
         DepthWork& W = e->depth[(size_t)d - 1];
         for (size_t i = 0; i < e->cases.size(); i++) {
             const lb_ctx* c = e->cases[i].c;
@@ -839,15 +818,7 @@ int engine_rebuild(lb_engine* e) {
                 (interior ? col : colb).push_back(w);
                 if (ddf) (interior ? tcol : tcolb).push_back(w);
             }
-            // ghost fill items: chunks of 256 entries (FP32), ghost blocks (16-bit)
-            const bool staged = e->storage != LB_STORAGE_FP32;
-            const int64_t n_items = staged ? (lev.ngent > 0 ? lev.ngh : 0) : (lev.ngent + 255) / 256;
-            if (l > 1)
-                for (int64_t q = 0; q < n_items; q++) {
-                    const int item = (int)(staged ? q : 256 * q);
-                    gh.push_back(mkwork(li, item, ci, nullptr));
-                    if (ddf) tgh.push_back(mkwork(li, item, ci, nullptr));
-                }
+            for (int32_t q = 0; q < lev.n_gchunks; q++) gh.push_back(mkwork(li, q, ci, (const int32_t*)(lev.gchunk + q)));
             for (const auto& ch : lev.lchunks) lk.push_back(mkwork(li, ch.first, ci, nullptr, ch.second));
             if (lev.wide) W.wide = 1;
             if (lev.wide_g) W.wide_g = 1;
@@ -858,12 +829,10 @@ int engine_rebuild(lb_engine* e) {
         RC(eupload(e, &W.gh, gh));
         RC(eupload(e, &W.lk, lk));
         RC(eupload(e, &W.tcol, tcol));
-        RC(eupload(e, &W.tgh, tgh));
         W.ncol = (int32_t)col.size();
         W.ngh = (int32_t)gh.size();
         W.nlk = (int32_t)lk.size();
         W.ntcol = (int32_t)tcol.size();
-        W.ntgh = (int32_t)tgh.size();
     }
     e->n_active = (int32_t)e->cases.size();
     e->dirty = false;
@@ -883,13 +852,12 @@ hipError_t engine_op(lb_engine* e, int d, int64_t j) {
     const lbk::CaseState* st = e->states;
     // one ghost pass per parent step fills the inputs of both child substeps
     const bool fill = (j & 1) == 0;
-    if (W.ngh && fill) ETRY(k->ghost_fill(e->las, st, W.gh, W.ngh, j, e->storage, 0, e->stream));
+    if (W.ngh && fill) ETRY(k->ghost_fill(e->las, st, W.gh, W.ngh, j, e->storage, e->stream));
     if (W.ncol)
         ETRY(k->collide(e->las, st, W.col, W.ncol, j, e->storage, W.wide, e->sched, e->waves, e->stream));
     if (W.ntcol) {
         // the thermal kernel has no persistent form
         const int tsched = e->sched == LB_SCHED_PERSISTENT ? LB_SCHED_LINEAR : e->sched;
-        if (W.ntgh && fill) ETRY(k->ghost_fill(e->las, st, W.tgh, W.ntgh, j, e->storage, 1, e->stream));
         ETRY(k->thermal(e->las, st, W.tcol, W.ntcol, j, e->storage, W.wide_g, tsched, e->stream));
     }
     if (W.nlk) ETRY(k->bouzidi(e->las, st, W.lk, W.nlk, j, e->storage, e->stream));
@@ -1153,7 +1121,7 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
     L.dx = d->dx;
     // Host tables: 0-based neighbour rows, block origins, and ghost blocks for
     // in-domain neighbour positions the level does not hold (levels > 1).
-    std::vector<int32_t> nbr((size_t)nb * Q), borg((size_t)nb * 3), gent;
+    std::vector<int32_t> nbr((size_t)nb * Q), borg((size_t)nb * 3);
     const int scale = 1 << (L.id - 1);
     const int64_t dbx = (int64_t)c->cfg.domain_nx * scale / 8, dby = (int64_t)c->cfg.domain_ny * scale / 8,
                   dbz = (int64_t)c->cfg.domain_nz * scale / 8;
@@ -1186,108 +1154,98 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
         borg[(size_t)b * 3 + 2] = (d->map_z[b] - 1) * 8;
     }
     const int32_t ngh = (int32_t)(gpos.size() / 3);
+    // The ghost fill's tables (GhostChunk, lb_kernels.h).  Ghost cell s serves
+    // direction k when s + c_k lies in a block of the level; which cells of a
+    // ghost block serve what follows from which of its 26 neighbours are real.
+    struct Served {
+        int m;                                             // group
+        uint32_t cells;                                    // its cells that serve any direction
+        std::vector<std::pair<int, uint32_t>> directions;  // direction, its cells that serve it
+        int64_t entries;                                   // number of those cells
+    };
+    std::unordered_map<uint32_t, std::vector<Served>> patterns;
+    auto pattern = [&patterns](uint32_t has_real) -> const std::vector<Served>& {
+        auto it = patterns.find(has_real);
+        if (it != patterns.end()) return it->second;
+        std::vector<Served> out;
+        for (int m = 0; m < 64; m++) {
+            Served v{m, 0u, {}, 0};
+            for (int k = 0; k < Q; k++) {
+                uint32_t cells = 0;
+                for (int d2 = 0; d2 < 8; d2++) {
+                    const int lx = 2 * (m & 3) + (d2 & 1), ly = 2 * ((m >> 2) & 3) + ((d2 >> 1) & 1),
+                              lz = 2 * (m >> 4) + (d2 >> 2);
+                    const int nx = lx + k % 3 - 1, ny = ly + (k / 3) % 3 - 1, nz = lz + k / 9 - 1;
+                    const int ox = nx < 0 ? -1 : (nx > 7 ? 1 : 0), oy = ny < 0 ? -1 : (ny > 7 ? 1 : 0),
+                              oz = nz < 0 ? -1 : (nz > 7 ? 1 : 0);
+                    if (ox == 0 && oy == 0 && oz == 0) continue;
+                    if (has_real & (1u << ((ox + 1) + 3 * (oy + 1) + 9 * (oz + 1)))) cells |= 1u << d2;
+                }
+                if (cells) v.directions.emplace_back(k, cells);
+                v.cells |= cells;
+            }
+            v.entries = __builtin_popcount(v.cells);
+            if (v.cells) out.push_back(std::move(v));
+        }
+        return patterns.emplace(has_real, std::move(out)).first->second;
+    };
+    std::vector<int32_t> gpb((size_t)ngh * 8, -1);
+    std::vector<uint32_t> ggroup, gpair;
+    std::vector<lbk::GhostChunk> gchunk;
+    lbk::GhostChunk ch{0, 0, 0, 0, 0};
+    int64_t n_entries = 0;
+    auto close_chunk = [&]() {
+        // a wave's work-items should read one direction of neighbouring groups
+        std::sort(gpair.begin() + ch.pair, gpair.end(), [](uint32_t u, uint32_t v) {
+            const uint32_t ku = (u >> 6) & 31u, kv = (v >> 6) & 31u;
+            return ku != kv ? ku < kv : (u & 63u) < (v & 63u);
+        });
+        if (ch.n_pairs > 0) gchunk.push_back(ch);
+    };
     for (int32_t g = 0; g < ngh; g++) {
         const int64_t px = gpos[(size_t)g * 3], py = gpos[(size_t)g * 3 + 1], pz = gpos[(size_t)g * 3 + 2];
-        borg.push_back((int32_t)((px - 1) * 8));
-        borg.push_back((int32_t)((py - 1) * 8));
-        borg.push_back((int32_t)((pz - 1) * 8));
-        // ghost cell s serves direction k when s + c_k lies in a block of the level
+        const int32_t origin[3] = {(int32_t)((px - 1) * 8), (int32_t)((py - 1) * 8), (int32_t)((pz - 1) * 8)};
+        borg.insert(borg.end(), origin, origin + 3);
+        // parent blocks that hold the 5^3 parent cells origin / 2 + 0..4 (1-based) of its corners
+        const Level& P = c->levels[(size_t)L.id - 2];
+        for (int s = 0; s < 8; s++) {
+            int b3[3];
+            bool in = true;
+            for (int ax = 0; ax < 3; ax++) {
+                b3[ax] = ((origin[ax] / 2 - 1) >> 3) + ((s >> ax) & 1);
+                in = in && b3[ax] >= 0 && b3[ax] < P.pd[ax];
+            }
+            if (!in) continue;
+            const int32_t pb =
+                P.grid_host[(size_t)b3[0] + (size_t)P.pd[0] * ((size_t)b3[1] + (size_t)P.pd[1] * (size_t)b3[2])];
+            if (pb >= (1 << 22)) return fail(c, LB_EINVAL, "level %d: parent block index %d too large", L.id, pb);
+            gpb[(size_t)g * 8 + (size_t)s] = pb;
+        }
         uint32_t has_real = 0;  // bit (ox+1) + 3(oy+1) + 9(oz+1): that neighbour block is real
         for (int n = 0; n < Q; n++)
             if (n != 13 && real.count(key(px + n % 3 - 1, py + (n / 3) % 3 - 1, pz + n / 9 - 1)))
                 has_real |= 1u << n;
-        for (int cl = 0; cl < NC && has_real != 0u; cl++) {
-            const int lx = cl & 7, ly = (cl >> 3) & 7, lz = cl >> 6;
-            uint32_t mask = 0;
-            for (int k = 0; k < Q; k++) {
-                const int nx = lx + k % 3 - 1, ny = ly + (k / 3) % 3 - 1, nz = lz + k / 9 - 1;
-                const int ox = nx < 0 ? -1 : (nx > 7 ? 1 : 0), oy = ny < 0 ? -1 : (ny > 7 ? 1 : 0),
-                          oz = nz < 0 ? -1 : (nz > 7 ? 1 : 0);
-                if (ox == 0 && oy == 0 && oz == 0) continue;
-                if (has_real & (1u << ((ox + 1) + 3 * (oy + 1) + 9 * (oz + 1)))) mask |= 1u << k;
+        for (const Served& v : pattern(has_real)) {
+            if (ch.n_groups == lbk::GHOST_GROUPS || ch.n_pairs + (int)v.directions.size() > lbk::GHOST_PAIRS ||
+                g - ch.ghost >= lbk::GHOST_BLOCKS) {
+                close_chunk();
+                ch = {g, (int32_t)ggroup.size(), (int32_t)gpair.size(), 0, 0};
             }
-            if (mask) {
-                gent.push_back((int32_t)(((nb + g) << 9) | cl));
-                gent.push_back((int32_t)mask);
-            }
+            const uint32_t gl = (uint32_t)(g - ch.ghost);
+            for (const auto& dir : v.directions)
+                gpair.push_back((uint32_t)ch.n_groups | (uint32_t)dir.first << 6 | dir.second << 11 | gl << 19);
+            uint32_t word = gl | (uint32_t)v.m << 5 | v.cells << 11;
+            for (int ax = 0; ax < 3; ax++)
+                word |= (uint32_t)((origin[ax] / 8) & 1) << (19 + ax) | (uint32_t)(origin[ax] == 0) << (22 + ax);
+            ggroup.push_back(word);
+            ch.n_groups++;
+            ch.n_pairs = (int16_t)(ch.n_pairs + (int)v.directions.size());
+            n_entries += v.entries;
         }
     }
+    close_chunk();
     L.ngh = ngh;
-    L.ngent = (int64_t)gent.size() / 2;
-    // The ghost fill's parent tables.  FP32 storage (ghost_kernel): per
-    // entry.  16-bit storage (ghost_kernel_staged): per ghost block.
-    const bool staged = c->cfg.storage != LB_STORAGE_FP32;
-    // The 8 parent cells of every ghost entry, as the interpolation of
-    // physics_interpolation.jl:4-127 addresses them: the fine cell centre at
-    // (g - 0.5) / 2 in parent cells, its lower corner clamped to the domain,
-    // each corner's parent block looked up in the parent grid (-1 where the
-    // parent level holds no block).  Static, so the kernel reads them instead
-    // of chasing the block origin and the parent grid per entry.
-    std::vector<int32_t> gpar(staged ? 0 : (size_t)L.ngent * 8, -1);
-    if (!staged && L.ngent > 0) {
-        const Level& P = c->levels[(size_t)L.id - 2];
-        const int pdx = P.pd[0], pdy = P.pd[1], pdz = P.pd[2];
-        for (int64_t e = 0; e < L.ngent; e++) {
-            const int gb = gent[(size_t)e * 2] >> 9, cl = gent[(size_t)e * 2] & 511;
-            const int fg[3] = {borg[(size_t)gb * 3 + 0] + (cl & 7) + 1, borg[(size_t)gb * 3 + 1] + ((cl >> 3) & 7) + 1,
-                               borg[(size_t)gb * 3 + 2] + (cl >> 6) + 1};
-            int lo[3], hi[3];
-            for (int ax = 0; ax < 3; ax++) {
-                const float pc = ((float)fg[ax] - 0.5f) * 0.5f;
-                lo[ax] = (int)std::floor(pc);
-                hi[ax] = lo[ax] + 1;
-                lo[ax] = std::max(1, lo[ax]);
-            }
-            for (int q = 0; q < 8; q++) {
-                const int pgx = (q & 1) ? hi[0] : lo[0], pgy = (q & 2) ? hi[1] : lo[1], pgz = (q & 4) ? hi[2] : lo[2];
-                const int pbx = (pgx - 1) / 8 + 1, pby = (pgy - 1) / 8 + 1, pbz = (pgz - 1) / 8 + 1;
-                if (pbx < 1 || pbx > pdx || pby < 1 || pby > pdy || pbz < 1 || pbz > pdz) continue;
-                const int32_t pb = P.grid_host[(size_t)(pbx - 1) + (size_t)pdx * ((size_t)(pby - 1) + (size_t)pdy * (pbz - 1))];
-                if (pb < 0) continue;
-                if (pb >= (1 << 22)) return fail(c, LB_EINVAL, "level %d: parent block index %d too large", L.id, pb);
-                const int cc = ((pgx - 1) % 8) + 8 * ((pgy - 1) % 8) + 64 * ((pgz - 1) % 8);
-                gpar[(size_t)e * 8 + q] = (pb << 9) | cc;
-            }
-        }
-    }
-    // Per ghost block, for the staged interpolation of physics_interpolation.jl:
-    // 4-127: its entries' range, the union of their served directions, and
-    // its parent region.  A fine cell at local index l (0..7) of a block with
-    // origin B (a multiple of 8) has its centre at (g - 0.5) / 2 in parent
-    // cells, g = B + l + 1; the interpolation's lower corner is
-    // max(1, B/2 + l/2) and its upper corner B/2 + l/2 + 1, so every corner
-    // of the block lies in the 5^3 parent cells B/2 + r, r = 0..4 per axis.
-    // gregion holds (parent block << 9 | cell) for those 125 cells, looked up
-    // in the parent grid, or -1 where the parent level holds no block (or the
-    // cell is outside it).
-    const int32_t ngs = staged && L.ngent > 0 ? ngh : 0;
-    std::vector<int32_t> gstart((size_t)ngs + (staged ? 1 : 0), 0), gregion((size_t)ngs * 125, -1);
-    std::vector<uint32_t> gbmask((size_t)ngs, 0u);
-    for (int64_t e = 0; e < (ngs > 0 ? L.ngent : 0); e++) {
-        const int g = (gent[(size_t)e * 2] >> 9) - nb;
-        gstart[(size_t)g + 1]++;
-        gbmask[(size_t)g] |= (uint32_t)gent[(size_t)e * 2 + 1];
-    }
-    for (int32_t g = 0; g < ngs; g++) gstart[(size_t)g + 1] += gstart[(size_t)g];
-    if (ngs > 0) {
-        const Level& P = c->levels[(size_t)L.id - 2];
-        const int pdx = P.pd[0], pdy = P.pd[1], pdz = P.pd[2];
-        for (int32_t g = 0; g < ngs; g++) {
-            int base[3];
-            for (int ax = 0; ax < 3; ax++) base[ax] = borg[(size_t)(nb + g) * 3 + ax] / 2;
-            for (int r = 0; r < 125; r++) {
-                const int pgx = base[0] + r % 5, pgy = base[1] + (r / 5) % 5, pgz = base[2] + r / 25;
-                if (pgx < 1 || pgy < 1 || pgz < 1) continue;
-                const int pbx = (pgx - 1) / 8 + 1, pby = (pgy - 1) / 8 + 1, pbz = (pgz - 1) / 8 + 1;
-                if (pbx > pdx || pby > pdy || pbz > pdz) continue;
-                const int32_t pb = P.grid_host[(size_t)(pbx - 1) + (size_t)pdx * ((size_t)(pby - 1) + (size_t)pdy * (pbz - 1))];
-                if (pb < 0) continue;
-                if (pb >= (1 << 22)) return fail(c, LB_EINVAL, "level %d: parent block index %d too large", L.id, pb);
-                const int cc = ((pgx - 1) % 8) + 8 * ((pgy - 1) % 8) + 64 * ((pgz - 1) % 8);
-                gregion[(size_t)g * 125 + r] = (pb << 9) | cc;
-            }
-        }
-    }
+    L.n_gchunks = (int32_t)gchunk.size();
     const size_t n4 = (size_t)nb * NC, n5 = ((size_t)nb + ngh) * NC * Q;
     L.wide = c->cfg.wide_offsets != 0 || (n5 + 512) * pop_bytes(c->cfg.storage) >= ((size_t)1 << 32);
     L.wide_g = L.wide;  // thermal populations use the same storage
@@ -1313,23 +1271,36 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
     RC(dalloc(c, &L.nbr, (size_t)nb * Q));
     RC(dalloc(c, &L.borg, borg.size()));
     RC(dalloc(c, &L.order, (size_t)nb));
-    RC(dalloc(c, &L.gent, gent.size()));
-    RC(dalloc(c, &L.gpar, gpar.size()));
-    if (!gstart.empty()) {
-        RC(dalloc(c, &L.gstart, gstart.size()));
-        RC(dalloc(c, &L.gregion, std::max<size_t>(gregion.size(), 1)));
-        RC(dalloc(c, &L.gbmask, std::max<size_t>(gbmask.size(), 1)));
+    const int64_t before_ghosts = c->bytes;
+    if (!gchunk.empty()) {
+        RC(dalloc(c, &L.gpb, gpb.size()));
+        RC(dalloc(c, &L.ggroup, ggroup.size()));
+        RC(dalloc(c, &L.gpair, gpair.size()));
+        RC(dalloc(c, &L.gchunk, gchunk.size()));
+        RC(h2d(c, L.gpb, gpb.data(), gpb.size()));
+        RC(h2d(c, L.ggroup, ggroup.data(), ggroup.size()));
+        RC(h2d(c, L.gpair, gpair.data(), gpair.size()));
+        RC(h2d(c, L.gchunk, gchunk.data(), gchunk.size()));
+    }
+    RC(ghost_list(c, L.id - 1, L));
+    // A case's footprint is a number that hosts plan with and keep (admission
+    // budgets, recorded sizes), so tables that got smaller leave it as it is.
+    // The ghost fill's was, per served cell and per ghost block, and with at
+    // least one element per table:
+    {
+        const int64_t e = n_entries, gh = n_entries > 0 ? ngh : 0;
+        const auto one = [](int64_t n) { return std::max<int64_t>(n, 1); };
+        const bool fp32 = c->cfg.storage == LB_STORAGE_FP32;
+        const int64_t work = (int64_t)sizeof(lbk::Work) * (fp32 ? (e + 255) / 256 : gh);
+        RC(keep_bytes(c, before_ghosts,
+                      4 * one(2 * e) + work +
+                          (fp32 ? 4 * one(8 * e) : 4 + 4 * (gh + 1) + 4 * one(125 * gh) + 4 * one(gh))));
     }
     const size_t ng = (size_t)d->ptr_dim_x * d->ptr_dim_y * d->ptr_dim_z;
     RC(dalloc(c, &L.grid, ng));
     L.pd[0] = d->ptr_dim_x;
     L.pd[1] = d->ptr_dim_y;
     L.pd[2] = d->ptr_dim_z;
-    if (!gent.empty()) RC(h2d(c, L.gent, gent.data(), gent.size()));
-    if (!gpar.empty()) RC(h2d(c, L.gpar, gpar.data(), gpar.size()));
-    if (!gstart.empty()) RC(h2d(c, L.gstart, gstart.data(), gstart.size()));
-    if (!gregion.empty()) RC(h2d(c, L.gregion, gregion.data(), gregion.size()));
-    if (!gbmask.empty()) RC(h2d(c, L.gbmask, gbmask.data(), gbmask.size()));
     if (nb > 0) {
         RC(h2d(c, L.nbr, nbr.data(), nbr.size()));
         RC(h2d(c, L.borg, borg.data(), borg.size()));
@@ -1387,13 +1358,9 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
     const int64_t before_links = c->bytes;
     RC(build_links(c, L, d));
     RC(link_list(c, L.id - 1, L));
-    // A case's footprint is a number that hosts plan with and keep (admission
-    // budgets, recorded sizes), so tables that got smaller leave it as it is:
-    // the links' 6 arrays (3 slots, 2 weights, 1 value) and chunks of 256.
+    // the footprint the links had: 6 arrays (3 slots, 2 weights, 1 value) and chunks of 256
     RC(keep_bytes(c, before_links,
                   L.nlinks * (3 * (L.lidx32 ? 4 : 8) + 12) + (L.nlinks + 255) / 256 * (int64_t)sizeof(lbk::Work)));
-    if (staged) RC(item_list(c, L.id - 1, L.ngent > 0 ? ngh : 0, &L.wgh, &L.n_gchunks));
-    else RC(chunk_list(c, L.id - 1, L.ngent, &L.wgh, &L.n_gchunks));
     RC(upload_level_args(c, L.id - 1));
     L.uploaded = true;
     return LB_OK;

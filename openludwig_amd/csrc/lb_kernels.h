@@ -66,6 +66,25 @@ struct BouzidiLinks {
     int32_t pad;
 };
 
+// Ghost fill.  The 2x2x2 cells 2m, 2m + 1 (per axis, m = 0..3) of a ghost
+// block interpolate from the same 8 parent cells: a group.  A pair is a group
+// and a direction that some of its cells serve.  A chunk is one work-group's
+// share: up to 32 groups and 256 pairs of up to 32 consecutive ghost blocks.
+//   group word: ghost - first (5 bits) | m = mx + 4 my + 16 mz (6) << 5 |
+//               its cells that serve any direction (8) << 11 | per axis, whether
+//               the block's first parent cell is the 5th of its parent block
+//               (3) << 19 and whether the block lies at the domain's low face
+//               (3) << 22
+//   pair word:  group - first (6) | direction (5) << 6 | its cells that serve
+//               it (8) << 11 | the group's ghost (5) << 19
+// (cell dx + 2 dy + 4 dz of a group is the local cell 2m + d)
+struct GhostChunk {
+    int32_t ghost, group, pair;  // first of the chunk
+    int16_t n_groups, n_pairs;
+};
+static_assert(sizeof(GhostChunk) == 16, "the kernel reads four words");
+constexpr int GHOST_GROUPS = 32, GHOST_PAIRS = 256, GHOST_BLOCKS = 32;
+
 struct LevelArgs {
     void* f[2];  // ping-pong pairs, indexed by substep parity (input = t_sub & 1)
     float* rho[2];
@@ -94,24 +113,14 @@ struct LevelArgs {
     const float* pvel[2];
     const void* pg[2];
     const float* pT[2];
-    const int32_t* pgrid;
-    int32_t pdx, pdy, pdz;
     float ptau, ptau_g;
-    // ghost entries: [n][2] = (ghost block << 9 | cell, 27-bit direction mask)
-    const int32_t* gent;
-    // FP32 storage, per ghost entry: its 8 parent cells (parent block << 9 |
-    // cell, or -1)
-    const int32_t* gpar;
-    // 16-bit storage (entries grouped by ghost block), per ghost block: its
-    // first entry ([ngh + 1]), its 125 parent cells (parent block << 9 |
-    // cell, or -1; cell r = rx + 5 ry + 25 rz of the parent region starting
-    // at half the block origin), the union of its entries' direction masks
-    const int32_t* gstart;
-    const int32_t* gregion;
-    const uint32_t* gbmask;
-    int64_t ngent;
+    // ghost fill: per ghost block the 8 parent blocks around it (-1 absent),
+    // and the chunks' groups and pairs (GhostChunk)
+    const int32_t* gpb;
+    const uint32_t* ggroup;
+    const uint32_t* gpair;
     BouzidiLinks links;
-    int64_t reserved[4];  // the record's size is part of a case's footprint
+    int64_t reserved[10];  // the record's size is part of a case's footprint
 };
 
 // Work list entry.  The neighbour row travels with the entry so that the
@@ -119,10 +128,11 @@ struct LevelArgs {
 // issued together.
 struct Work {
     int32_t li;              // LevelArgs index
-    int32_t item;            // block (stream-collide), first entry of a chunk, or ghost block
+    int32_t item;            // block (stream-collide) or first link of a chunk
     int32_t ci;              // CaseState index
     int32_t flags;           // stream-collide: WORK_* of the block; links: entries of the chunk
-    const int32_t* nbr_row;  // the block's neighbour row (stream-collide), else null
+    // stream-collide: the block's neighbour row; ghost fill: the GhostChunk; else null
+    const int32_t* nbr_row;
 };
 // some neighbour of the block is neither a block nor a ghost block (domain boundary)
 constexpr int32_t WORK_BOUNDARY = 8;
@@ -195,7 +205,7 @@ struct FiniteEntry {
     hipError_t thermal(const lbk::LevelArgs* las, const lbk::CaseState* states, const lbk::Work* work,    \
                        int32_t n_tiles, int64_t j, int storage, int wide, int sched, hipStream_t s);     \
     hipError_t ghost_fill(const lbk::LevelArgs* las, const lbk::CaseState* states, const lbk::Work* work, int32_t n_chunks, int64_t j,  \
-                          int storage, int thermal, hipStream_t s);                                      \
+                          int storage, hipStream_t s);                                                   \
     hipError_t bouzidi(const lbk::LevelArgs* las, const lbk::CaseState* states, const lbk::Work* work, int32_t n_chunks, int64_t j,     \
                        int storage, hipStream_t s);                                                      \
     hipError_t set_state(lbk::CaseState* st, const lbk::CaseState& v, hipStream_t s);                   \

@@ -98,17 +98,9 @@ struct ThermalArgs {
 struct GhostArgs {
     void* f;   // input half of substep j (ghost blocks at index >= nb)
     void* f2;  // input half of substep j + 1
-    const int32_t* entries;
-    const int32_t* parents;  // [n][8] parent cells of each entry (LevelArgs::gpar)
-    int64_t n;
     const void* a_new;
-    const float* s_new;
-    const float* u_new;
     const void* a_old;
-    const float* s_old;
-    const float* u_old;
     float tau_fine, tau_coarse;
-    int32_t temporal, comp, thermal;
 };
 
 // The case record, read through the global address space (uniform loads, in
@@ -228,26 +220,15 @@ __device__ __forceinline__ ThermalArgs thermal_view(const LevelArgs& L, const Ca
 // step) is "old".  The temporal weight is 0 for the first child substep and
 // 0.5 for the second (solver_control.jl:66-96); f and f2 are their input
 // halves.
-__device__ __forceinline__ GhostArgs ghost_view(const LevelArgs& L, const CaseState& S, int64_t j, int thermal) {
-    const int par = (int)(substep(L, S, j) & 1);
-    const int ppar = (int)(((S.t0 << (L.lshift - 1)) + (j >> 1)) & 1);
+__device__ __forceinline__ GhostArgs ghost_view(const LevelArgs& L, int par, int ppar, bool temporal, bool thermal) {
     GhostArgs g;
+    const int po = temporal ? ppar : 1 - ppar;
     g.f = thermal ? (void*)L.g[par] : L.f[par];
     g.f2 = thermal ? (void*)L.g[1 - par] : L.f[1 - par];
-    g.entries = L.gent;
-    g.n = L.ngent;
-    g.parents = L.gpar;
     g.a_new = thermal ? (const void*)L.pg[1 - ppar] : L.pf[1 - ppar];
-    g.s_new = thermal ? L.pT[1 - ppar] : L.prho[1 - ppar];
-    g.u_new = L.pvel[1 - ppar];
-    g.a_old = thermal ? (const void*)L.pg[ppar] : L.pf[ppar];
-    g.s_old = thermal ? L.pT[ppar] : L.prho[ppar];
-    g.u_old = L.pvel[ppar];
+    g.a_old = thermal ? (const void*)L.pg[po] : L.pf[po];
     g.tau_fine = thermal ? L.tau_g : L.tau;
     g.tau_coarse = thermal ? L.ptau_g : L.ptau;
-    g.temporal = S.temporal;
-    g.comp = S.comp;
-    g.thermal = thermal;
     return g;
 }
 
@@ -262,6 +243,7 @@ __device__ __forceinline__ const __attribute__((address_space(1))) int32_t* gp(c
     return (const __attribute__((address_space(1))) int32_t*)p;
 }
 typedef __attribute__((address_space(1))) uint16_t GU16;
+typedef __attribute__((address_space(1))) uint32_t GU32;
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) v4u GV4U;
 typedef __attribute__((address_space(1))) char GC;
@@ -289,6 +271,11 @@ struct Codec<0> {
     static __device__ __forceinline__ void stream(void* base, size_t i, float f, float) {
         __builtin_nontemporal_store(f, &((GF*)base)[i]);
     }
+    // two consecutive values, the first at an even slot
+    static __device__ __forceinline__ void store2(void* base, size_t i, float f0, float f1, float) {
+        typedef float v2f __attribute__((ext_vector_type(2)));
+        *(__attribute__((address_space(1))) v2f*)((GF*)base + i) = v2f{f0, f1};
+    }
     // the stored bits of f (for the staged stores of stream_tile)
     static __device__ __forceinline__ uint32_t bits(float f, float) { return __float_as_uint(f); }
 };
@@ -312,6 +299,9 @@ struct Codec<1> {
     }
     static __device__ __forceinline__ uint16_t bits(float f, float w) {
         return (uint16_t)__half_as_ushort(__float2half_rn(f - w));
+    }
+    static __device__ __forceinline__ void store2(void* base, size_t i, float f0, float f1, float w) {
+        *(GU32*)((GU16*)base + i) = (uint32_t)bits(f0, w) | (uint32_t)bits(f1, w) << 16;
     }
 };
 template <>
@@ -339,6 +329,9 @@ struct Codec<2> {
         __builtin_nontemporal_store(enc(f - w), &((GU16*)base)[i]);
     }
     static __device__ __forceinline__ uint16_t bits(float f, float w) { return enc(f - w); }
+    static __device__ __forceinline__ void store2(void* base, size_t i, float f0, float f1, float w) {
+        *(GU32*)((GU16*)base + i) = (uint32_t)bits(f0, w) | (uint32_t)bits(f1, w) << 16;
+    }
 };
 
 // Staged stores of a wave's stream-collide outputs.  A wave is one z-plane
@@ -1331,72 +1324,6 @@ hipError_t thermal(const LevelArgs* las, const CaseState* states, const Work* wo
     return hipGetLastError();
 }
 
-// Parent population component k at the 8 corners (new and, with temporal
-// interpolation, old), decoded to FP32.
-template <int ST>
-__device__ __forceinline__ void ghost_load(const GhostArgs& a, int k, const bool* ok, const int* cb, const int* cc,
-                                           bool need_old, float* ln, float* lo) {
-    const float w_k = wk_rt(k);
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-        ln[q] = 0.0f;
-        lo[q] = 0.0f;
-        if (ok[q]) {
-            ln[q] = Codec<ST>::load(a.a_new, fidx(cb[q], k, cc[q]), w_k);
-            if (need_old) lo[q] = Codec<ST>::load(a.a_old, fidx(cb[q], k, cc[q]), w_k);
-        }
-    }
-}
-
-// Temporal and trilinear blend of component k for both child substeps,
-// rescaled non-equilibrium part, stored into both input halves.
-template <int ST>
-__device__ __forceinline__ void ghost_blend_store(const GhostArgs& a, int k, const bool* ok, const float* ln,
-                                                  const float* lo, bool use_old0, bool use_old1, float wx, float wy,
-                                                  float wz, const float* r0, const float* r1, float scale, int gb,
-                                                  int c) {
-    const float tw0 = 0.0f, tw1 = 0.5f;
-    const float w_k = wk_rt(k), cx = (float)CX(k), cy = (float)CY(k), cz = (float)CZ(k);
-    float f0[8], f1[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++) {
-        if (ok[q]) {
-            const float fn = ln[q], fo_ = lo[q];
-            f0[q] = use_old0 ? fo_ * (1.0f - tw0) + fn * tw0 : fn;
-            f1[q] = use_old1 ? fo_ * (1.0f - tw1) + fn * tw1 : fn;
-        } else {
-            f0[q] = q == 0 ? w_k : f0[0];
-            f1[q] = q == 0 ? w_k : f1[0];
-        }
-    }
-    float rr0, rr1;
-    {
-        float c00 = f0[0] * (1.0f - wx) + f0[1] * wx;
-        float c01 = f0[4] * (1.0f - wx) + f0[5] * wx;
-        float c10 = f0[2] * (1.0f - wx) + f0[3] * wx;
-        float c11 = f0[6] * (1.0f - wx) + f0[7] * wx;
-        float c0 = c00 * (1.0f - wy) + c10 * wy;
-        float c1 = c01 * (1.0f - wy) + c11 * wy;
-        rr0 = c0 * (1.0f - wz) + c1 * wz;
-    }
-    {
-        float c00 = f1[0] * (1.0f - wx) + f1[1] * wx;
-        float c01 = f1[4] * (1.0f - wx) + f1[5] * wx;
-        float c10 = f1[2] * (1.0f - wx) + f1[3] * wx;
-        float c11 = f1[6] * (1.0f - wx) + f1[7] * wx;
-        float c0 = c00 * (1.0f - wy) + c10 * wy;
-        float c1 = c01 * (1.0f - wy) + c11 * wy;
-        rr1 = c0 * (1.0f - wz) + c1 * wz;
-    }
-    const float eq0 = a.thermal ? geq(r0[0], r0[1], r0[2], r0[3], w_k, cx, cy, cz)
-                                : feq_auto(r0[0], r0[1], r0[2], r0[3], w_k, cx, cy, cz, a.comp);
-    const float eq1 = a.thermal ? geq(r1[0], r1[1], r1[2], r1[3], w_k, cx, cy, cz)
-                                : feq_auto(r1[0], r1[1], r1[2], r1[3], w_k, cx, cy, cz, a.comp);
-    const float neq0 = rr0 - eq0, neq1 = rr1 - eq1;
-    Codec<ST>::store(a.f, fidx(gb, k, c), eq0 + neq0 * scale, w_k);
-    Codec<ST>::store(a.f2, fidx(gb, k, c), eq1 + neq1 * scale, w_k);
-}
-
 // ---------------------------------------------------------------------------
 // Ghost-cell interpolation: interpolate_with_rescaling / its thermal twin
 // (physics_interpolation.jl:4-127, 135-248) for every direction a ghost cell
@@ -1405,113 +1332,123 @@ __device__ __forceinline__ void ghost_blend_store(const GhostArgs& a, int k, con
 // one pass, run before the first substep, computes both: the tw = 0 values go
 // to the ghost slots of the first substep's input half, the tw = 0.5 values to
 // the other half, which the first substep does not write (its collide writes
-// real blocks only).  The corner geometry and the density/velocity part of
-// the trilinear blend depend on the cell only and are computed once; each
-// direction then blends its own population component.  Per value, the
-// operations are those of the reference function, in its order.
-template <int ST>
-__global__ void __launch_bounds__(256) ghost_kernel(const LevelArgs* __restrict__ las,
-                                                    const CaseState* __restrict__ states,
-                                                    const Work* __restrict__ work, int64_t j, int thermal) {
-    const Work wk = work[blockIdx.x];
-    const LevelArgs& L = las[wk.li];
-    const CaseState S = case_state(states + wk.ci);
-    if (!live(L, S, j)) return;
-    const GhostArgs a = ghost_view(L, S, j, thermal);
-    const int64_t i = (int64_t)wk.item + threadIdx.x;
-    if (i >= a.n) return;
-    const int e0 = a.entries[2 * i];
-    const uint32_t mask = (uint32_t)a.entries[2 * i + 1];
-    const int gb = e0 >> 9, c = e0 & 511;
-    // The fine cell centre lies at (g - 0.5) / 2 in parent cells, g = block
-    // origin (a multiple of 8) + local index + 1, so its fractional part is
-    // 0.25 for an even local index and 0.75 for an odd one (exactly what
-    // (g - 0.5) * 0.5 - floor(...) gives in FP32).  The 8 parent cells come
-    // precomputed with the entry.
-    const float wx = (c & 1) ? 0.75f : 0.25f;
-    const float wy = ((c >> 3) & 1) ? 0.75f : 0.25f;
-    const float wz = ((c >> 6) & 1) ? 0.75f : 0.25f;
-    int par[8];
-    {
-        typedef int32_t v4i __attribute__((ext_vector_type(4)));
-        const __attribute__((address_space(1))) v4i* pp =
-            (const __attribute__((address_space(1))) v4i*)(a.parents + 8 * i);
-        const v4i p0 = pp[0], p1 = pp[1];
-        par[0] = p0.x, par[1] = p0.y, par[2] = p0.z, par[3] = p0.w;
-        par[4] = p1.x, par[5] = p1.y, par[6] = p1.z, par[7] = p1.w;
+// real blocks only).  Per value, the operations are those of the reference
+// function, in its order.
+//
+// Bound by the gathers from the parent (8 cells, new and old, per value).  The
+// 2x2x2 fine cells of a group share their 8 parent cells, so a work-item loads
+// a component of a group once for all of its cells (4 on a face): first the
+// density and velocity blends of the chunk's groups into LDS, a work-item per
+// (group, field), then a work-item per (group, direction).  Against a
+// work-item per ghost cell (FP32) and per-block staging of the 5^3 parent
+// region in LDS (16-bit), one launch of the finest fill: 22.8 -> 16.0 us (FP32
+// sphere, 500 chunks), 44.5 -> 34.4 us (6.1 M-cell cube), 142 -> 123 us (52.5
+// M cells); FP16 39.6 -> 22.7 us (ellipsoid), and on the 10.7 M-cell thermal
+// wing 2 x 65.6 -> 76 us for f and g in one launch.  The two cells of an x row
+// in one store did not change it; 8 waves per SIMD (32 groups of LDS) gave up to
+// 1 % of a step over 7.
+// Parent cell of corner q of a group, as (block << 9 | cell) or -1.  Per axis,
+// the fine cell centres lie at (x - 0.5) / 2 in parent cells, x = origin +
+// local + 1, so the lower corner is max(1, origin / 2 + m) and the upper one
+// origin / 2 + m + 1 (1-based); origin / 2 is a multiple of 4.  gpb holds the
+// parent blocks of the two that origin / 2 - 1 and its successors lie in.
+__device__ __forceinline__ int ghost_corner(const LevelArgs& L, int first, uint32_t grp, int q) {
+    int slot = 0, cell = 0;
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++) {
+        const int m = (int)((grp >> (5 + 2 * ax)) & 3u);
+        const int half = (int)((grp >> (19 + ax)) & 1u) * 4;  // origin / 2 within its parent block
+        const bool low = ((grp >> (22 + ax)) & 1u) != 0u;
+        // 0-based: lower half + m - 1, upper half + m; -1 is the block before
+        int x = half + m - 1 + ((q >> ax) & 1);
+        if (low && x < 0) x = 0;
+        slot |= (half == 0 && x >= 0 ? 1 : 0) << ax;
+        cell |= (x & 7) << (3 * ax);
     }
-    // temporal blend with tw = 0 (substep j) and tw = 0.5 (substep j + 1)
-    const bool use_old0 = a.temporal == 1 && 0.0f < 0.99f;
-    const bool use_old1 = a.temporal == 1 && 0.5f < 0.99f;
+    const int pb = gp(L.gpb)[(size_t)(first + (int)(grp & 31u)) * 8 + slot];
+    return pb < 0 ? -1 : (pb << 9) | cell;
+}
+
+// Trilinear blend of the 8 corner values with the weights of one fine cell.
+__device__ __forceinline__ float ghost_blend(const float (&v)[8], float wx, float wy, float wz) {
+    float c00 = v[0] * (1.0f - wx) + v[1] * wx;
+    float c01 = v[4] * (1.0f - wx) + v[5] * wx;
+    float c10 = v[2] * (1.0f - wx) + v[3] * wx;
+    float c11 = v[6] * (1.0f - wx) + v[7] * wx;
+    float c0 = c00 * (1.0f - wy) + c10 * wy;
+    float c1 = c01 * (1.0f - wy) + c11 * wy;
+    return c0 * (1.0f - wz) + c1 * wz;
+}
+
+// Temporal blends (tw = 0 and 0.5) of one field's corner values; a corner the
+// parent level does not hold takes the first corner's value, a missing first
+// corner `rest`.
+__device__ __forceinline__ void ghost_in_time(const int (&at)[8], const float (&vn)[8], const float (&vo)[8],
+                                              bool temporal, float rest, float (&v0)[8], float (&v1)[8]) {
     const float tw0 = 0.0f, tw1 = 0.5f;
-    int cb[8], cc[8];
-    bool ok[8];
-    float v0[8][4], v1[8][4];
 #pragma unroll
     for (int q = 0; q < 8; q++) {
-        ok[q] = par[q] >= 0;
-        cb[q] = ok[q] ? (par[q] >> 9) : 0;
-        cc[q] = ok[q] ? (par[q] & 511) : 0;
-        if (ok[q]) {
-            const size_t i4 = (size_t)cb[q] * NC + cc[q];
-            const size_t iv = (size_t)cb[q] * 3 * NC + cc[q];
-            const float rn = a.s_new[i4], uxn = a.u_new[iv], uyn = a.u_new[iv + NC], uzn = a.u_new[iv + 2 * NC];
-            float ro = 0.0f, uxo = 0.0f, uyo = 0.0f, uzo = 0.0f;
-            if (use_old0 || use_old1) {
-                ro = a.s_old[i4];
-                uxo = a.u_old[iv];
-                uyo = a.u_old[iv + NC];
-                uzo = a.u_old[iv + 2 * NC];
-            }
-            if (use_old0) {
-                v0[q][0] = ro * (1.0f - tw0) + rn * tw0;
-                v0[q][1] = uxo * (1.0f - tw0) + uxn * tw0;
-                v0[q][2] = uyo * (1.0f - tw0) + uyn * tw0;
-                v0[q][3] = uzo * (1.0f - tw0) + uzn * tw0;
-            } else {
-                v0[q][0] = rn; v0[q][1] = uxn; v0[q][2] = uyn; v0[q][3] = uzn;
-            }
-            if (use_old1) {
-                v1[q][0] = ro * (1.0f - tw1) + rn * tw1;
-                v1[q][1] = uxo * (1.0f - tw1) + uxn * tw1;
-                v1[q][2] = uyo * (1.0f - tw1) + uyn * tw1;
-                v1[q][3] = uzo * (1.0f - tw1) + uzn * tw1;
-            } else {
-                v1[q][0] = rn; v1[q][1] = uxn; v1[q][2] = uyn; v1[q][3] = uzn;
-            }
-        } else if (q == 0) {
-            v0[0][0] = 1.0f; v0[0][1] = 0.0f; v0[0][2] = 0.0f; v0[0][3] = 0.0f;
-            v1[0][0] = 1.0f; v1[0][1] = 0.0f; v1[0][2] = 0.0f; v1[0][3] = 0.0f;
-        } else {
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                v0[q][m] = v0[0][m];
-                v1[q][m] = v1[0][m];
-            }
-        }
+        const float b0 = temporal ? vo[q] * (1.0f - tw0) + vn[q] * tw0 : vn[q];
+        const float b1 = temporal ? vo[q] * (1.0f - tw1) + vn[q] * tw1 : vn[q];
+        v0[q] = at[q] >= 0 ? b0 : (q == 0 ? rest : v0[0]);
+        v1[q] = at[q] >= 0 ? b1 : (q == 0 ? rest : v1[0]);
     }
-    float r0[4], r1[4];
+}
+
+// The weights of cell d (dx + 2 dy + 4 dz) of a group: the fractional part of
+// its centre in parent cells is 0.25 for an even local index, 0.75 for an odd
+// one (exactly what (x - 0.5) * 0.5 - floor(...) gives in FP32).
+__device__ __forceinline__ float ghost_weight(int d, int ax) { return ((d >> ax) & 1) ? 0.75f : 0.25f; }
+
+// Component k at the 8 corners, new and old (without temporal interpolation
+// the view's old half is the new one); a missing corner reads slot 0, unused.
+template <int ST>
+__device__ __forceinline__ void ghost_load(const GhostArgs& a, const int (&at)[8], int k, float (&vn)[8],
+                                           float (&vo)[8]) {
+    const float w_k = wk_rt(k);
 #pragma unroll
-    for (int m = 0; m < 4; m++) {
-        {
-            float c00 = v0[0][m] * (1.0f - wx) + v0[1][m] * wx;
-            float c01 = v0[4][m] * (1.0f - wx) + v0[5][m] * wx;
-            float c10 = v0[2][m] * (1.0f - wx) + v0[3][m] * wx;
-            float c11 = v0[6][m] * (1.0f - wx) + v0[7][m] * wx;
-            float c0 = c00 * (1.0f - wy) + c10 * wy;
-            float c1 = c01 * (1.0f - wy) + c11 * wy;
-            r0[m] = c0 * (1.0f - wz) + c1 * wz;
-        }
-        {
-            float c00 = v1[0][m] * (1.0f - wx) + v1[1][m] * wx;
-            float c01 = v1[4][m] * (1.0f - wx) + v1[5][m] * wx;
-            float c10 = v1[2][m] * (1.0f - wx) + v1[3][m] * wx;
-            float c11 = v1[6][m] * (1.0f - wx) + v1[7][m] * wx;
-            float c0 = c00 * (1.0f - wy) + c10 * wy;
-            float c1 = c01 * (1.0f - wy) + c11 * wy;
-            r1[m] = c0 * (1.0f - wz) + c1 * wz;
-        }
+    for (int q = 0; q < 8; q++) {
+        const size_t i = at[q] >= 0 ? fidx(at[q] >> 9, k, at[q] & 511) : 0;
+        vn[q] = Codec<ST>::load(a.a_new, i, w_k);
+        vo[q] = Codec<ST>::load(a.a_old, i, w_k);
     }
+}
+
+// One field of a group blended for each of its cells, tw = 0 and (half floats
+// on) tw = 0.5.
+__device__ __forceinline__ void ghost_field(const float* fn, const float* fo, int per, const int32_t (&s_at)[8],
+                                            uint32_t cells, bool temporal, float rest, float* mac, int stride,
+                                            int half) {
+    int ga[8];
+    float un[8], uo[8], v0[8], v1[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+        ga[q] = s_at[q];
+        const size_t i = ga[q] >= 0 ? (size_t)(ga[q] >> 9) * per + (ga[q] & 511) : 0;
+        un[q] = gp(fn)[i];
+        uo[q] = gp(fo)[i];
+    }
+    ghost_in_time(ga, un, uo, temporal, rest, v0, v1);
+#pragma unroll 1
+    for (; cells != 0u; cells &= cells - 1u) {
+        const int d = __builtin_ctz(cells);
+        const float wx = ghost_weight(d, 0), wy = ghost_weight(d, 1), wz = ghost_weight(d, 2);
+        mac[d * stride] = ghost_blend(v0, wx, wy, wz);
+        mac[d * stride + half] = ghost_blend(v1, wx, wy, wz);
+    }
+}
+
+// Interpolated component k of the cells of one pair, rescaled in its
+// non-equilibrium part, into both input halves.
+template <int ST, bool THERMAL>
+__device__ __forceinline__ void ghost_store(const GhostArgs& a, const float4 (*mac)[2], const float (*mact)[2],
+                                            uint32_t pair,
+                                            uint32_t grp, int gb, const int (&at)[8], const float (&vn)[8], const float (&vo)[8],
+                                            bool temporal, int comp) {
+    const int lg = (int)(pair & 63u), k = (int)((pair >> 6) & 31u), m = (int)((grp >> 5) & 63u);
+    const float w_k = wk_rt(k), cx = (float)CX(k), cy = (float)CY(k), cz = (float)CZ(k);
+    float f0[8], f1[8];
+    ghost_in_time(at, vn, vo, temporal, w_k, f0, f1);
     const float tc = a.tau_coarse - 0.5f;
     const float tf = a.tau_fine - 0.5f;
     float scale = 1.0f;
@@ -1519,232 +1456,117 @@ __global__ void __launch_bounds__(256) ghost_kernel(const LevelArgs* __restrict_
         scale = tf / tc;
         scale = scale > 100.0f ? 100.0f : (scale < 0.01f ? 0.01f : scale);
     }
-    const bool need_old = use_old0 || use_old1;
-    if constexpr (ST == 0) {
-        // FP32: the parent values of the next served direction are loaded
-        // while the current one is blended (ghost time -21 % on the cube
-        // case).  The 16-bit forms keep the plain loop below, whose higher
-        // occupancy hides their short loads better (pipelined: +9 %).
-        uint32_t m = mask;
-        int k = m ? __builtin_ctz(m) : -1;
-        float ln[8], lo[8];
-        if (k >= 0) ghost_load<ST>(a, k, ok, cb, cc, need_old, ln, lo);
-        while (k >= 0) {
-            m &= m - 1u;
-            const int kn = m ? __builtin_ctz(m) : -1;
-            float nn[8], no[8];
-            if (kn >= 0) ghost_load<ST>(a, kn, ok, cb, cc, need_old, nn, no);
-            ghost_blend_store<ST>(a, k, ok, ln, lo, use_old0, use_old1, wx, wy, wz, r0, r1, scale, gb, c);
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                ln[q] = nn[q];
-                lo[q] = no[q];
-            }
-            k = kn;
-        }
-    } else {
+    // The two cells of an x row leave in one store (whole 32-byte sectors with
+    // the neighbouring groups' rows).
 #pragma unroll 1
-        for (int k = 0; k < 27; k++) {
-            if (!(mask & (1u << k))) continue;
-            float ln[8], lo[8];
-            ghost_load<ST>(a, k, ok, cb, cc, need_old, ln, lo);
-            ghost_blend_store<ST>(a, k, ok, ln, lo, use_old0, use_old1, wx, wy, wz, r0, r1, scale, gb, c);
+    for (int row = 0; row < 4; row++) {  // dy + 2 dz
+        const uint32_t bits = (pair >> (11 + 2 * row)) & 3u;
+        if (bits == 0u) continue;
+        const float wy = (row & 1) ? 0.75f : 0.25f, wz = (row & 2) ? 0.75f : 0.25f;
+        float out0[2], out1[2];
+#pragma unroll
+        for (int dx = 0; dx < 2; dx++) {
+            out0[dx] = out1[dx] = 0.0f;
+            if (bits & (1u << dx)) {
+                const int d = dx + 2 * row;
+                const float wx = ghost_weight(d, 0);
+                const float rr0 = ghost_blend(f0, wx, wy, wz), rr1 = ghost_blend(f1, wx, wy, wz);
+                const float4 r0 = mac[lg * 8 + d][0], r1 = mac[lg * 8 + d][1];  // density, velocity
+                float eq0, eq1;
+                if constexpr (THERMAL) {
+                    eq0 = geq(mact[lg * 8 + d][0], r0.y, r0.z, r0.w, w_k, cx, cy, cz);
+                    eq1 = geq(mact[lg * 8 + d][1], r1.y, r1.z, r1.w, w_k, cx, cy, cz);
+                } else {
+                    eq0 = feq_auto(r0.x, r0.y, r0.z, r0.w, w_k, cx, cy, cz, comp);
+                    eq1 = feq_auto(r1.x, r1.y, r1.z, r1.w, w_k, cx, cy, cz, comp);
+                }
+                const float neq0 = rr0 - eq0, neq1 = rr1 - eq1;
+                out0[dx] = eq0 + neq0 * scale;
+                out1[dx] = eq1 + neq1 * scale;
+            }
+        }
+        const int c = 2 * (m & 3) + 8 * (2 * ((m >> 2) & 3) + (row & 1)) + 64 * (2 * (m >> 4) + (row >> 1));
+        const size_t i = fidx(gb, k, c);
+        if (bits == 3u) {
+            Codec<ST>::store2(a.f, i, out0[0], out0[1], w_k);
+            Codec<ST>::store2(a.f2, i, out1[0], out1[1], w_k);
+        } else {
+            const int dx = (int)(bits >> 1);
+            Codec<ST>::store(a.f, i + dx, dx ? out0[1] : out0[0], w_k);
+            Codec<ST>::store(a.f2, i + dx, dx ? out1[1] : out1[0], w_k);
         }
     }
 }
-
-// 16-bit storage: one work-group per ghost block.  Every interpolation
-// corner of the block's cells lies in a 5^3 region of parent cells
-// (LevelArgs::gregion), so the work-group first stages that region in LDS:
-// the parent density (or temperature) and velocity, new and old, and the
-// parent populations of the directions the block serves (gbmask), decoded to
-// FP32, 125 cells per direction and time level, the consecutive work-items of
-// a load taking consecutive cells of a parent row.  Each work-item then
-// interpolates its entries from LDS, with the operations of ghost_kernel in
-// its order.  Measured on the 52.5M-cell cube case: FP16 step -1.0 % (A/B on
-// one box); in FP32 the per-entry kernel above, which loads the next
-// direction's corners while blending the current one, stays faster (fill
-// 103 us against 114 us per launch).
-constexpr int GREG = 125;  // parent cells of a ghost block's region
 
 template <int ST>
-__global__ void __launch_bounds__(256) ghost_kernel_staged(const LevelArgs* __restrict__ las,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) ghost_kernel(const LevelArgs* __restrict__ las,
                                                     const CaseState* __restrict__ states,
-                                                    const Work* __restrict__ work, int64_t j, int thermal) {
-    __shared__ float spop[27 * 2 * GREG];  // [direction slot][new, old][region cell]
-    __shared__ float smac[8 * GREG];       // [new rho/T, ux, uy, uz, old rho/T, ux, uy, uz][region cell]
-    __shared__ int32_t sreg[GREG];
+                                                    const Work* __restrict__ work, int64_t j) {
+    __shared__ float4 mac[GHOST_GROUPS * 8][2];  // [cell of group][tw = 0, 0.5]: density, velocity
+    __shared__ float mact[GHOST_GROUPS * 8][2];  // temperature
+    __shared__ int32_t s_at[GHOST_GROUPS][8];                   // parent cells of the groups' corners
+    __shared__ uint32_t s_grp[GHOST_GROUPS];
     const Work wk = work[blockIdx.x];
     const LevelArgs& L = las[wk.li];
+    const auto* cw = gp(wk.nbr_row);
+    const int sizes = cw[3];
+    const struct { int ghost, group, pair, n_groups, n_pairs; } ch = {cw[0], cw[1], cw[2], sizes & 0xffff, sizes >> 16};
     const CaseState S = case_state(states + wk.ci);
     if (!live(L, S, j)) return;
-    const GhostArgs a = ghost_view(L, S, j, thermal);
-    const int g = wk.item;
     const int tid = (int)threadIdx.x;
-    const uint32_t bmask = L.gbmask[g];
-    // temporal blend with tw = 0 (substep j) and tw = 0.5 (substep j + 1)
-    const bool use_old0 = a.temporal == 1 && 0.0f < 0.99f;
-    const bool use_old1 = a.temporal == 1 && 0.5f < 0.99f;
-    const bool need_old = use_old0 || use_old1;
-    const float tw0 = 0.0f, tw1 = 0.5f;
-    if (tid < GREG) sreg[tid] = L.gregion[(size_t)g * GREG + tid];
+    // the parent's last step is substep j >> 1 of the parent level
+    const int par = (int)(substep(L, S, j) & 1);
+    const int ppar = (int)(((S.t0 << (L.lshift - 1)) + (j >> 1)) & 1);
+    const bool temporal = S.temporal == 1;
+    const bool ddf = L.g[0] != nullptr;
+    const GhostArgs a = ghost_view(L, par, ppar, temporal, false);
+    typedef const __attribute__((address_space(1))) uint32_t GW;
+    // the parent cells of the chunk's groups
+    for (int t = tid; t < 8 * ch.n_groups; t += 256) {
+        const uint32_t grp = ((GW*)L.ggroup)[ch.group + (t >> 3)];
+        s_at[t >> 3][t & 7] = ghost_corner(L, ch.ghost, grp, t & 7);
+        if ((t & 7) == 0) s_grp[t >> 3] = grp;
+    }
+    const uint32_t pair = tid < ch.n_pairs ? ((GW*)L.gpair)[ch.pair + tid] : 0u;
     __syncthreads();
-    // stage the parent region
-    if (tid < GREG) {
-        const int p = sreg[tid];
-        float m[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        if (p >= 0) {
-            const size_t i4 = (size_t)(p >> 9) * NC + (p & 511);
-            const size_t iv = (size_t)(p >> 9) * 3 * NC + (p & 511);
-            m[0] = a.s_new[i4], m[1] = a.u_new[iv], m[2] = a.u_new[iv + NC], m[3] = a.u_new[iv + 2 * NC];
-            if (need_old) {
-                m[4] = a.s_old[i4];
-                m[5] = a.u_old[iv];
-                m[6] = a.u_old[iv + NC];
-                m[7] = a.u_old[iv + 2 * NC];
-            }
-        }
+    // the pair's corner values are on their way while the fields are blended
+    const int k = (int)((pair >> 6) & 31u);
+    int at[8];
+    float vn[8], vo[8];
 #pragma unroll
-        for (int q = 0; q < 8; q++) smac[q * GREG + tid] = m[q];
+    for (int q = 0; q < 8; q++) at[q] = s_at[pair & 63u][q];
+    ghost_load<ST>(a, at, k, vn, vo);
+    const int po = temporal ? ppar : 1 - ppar;
+    if (tid < 4 * ch.n_groups) {
+        const int lg = tid >> 2, m = tid & 3;
+        const float* fn = m == 0 ? L.prho[1 - ppar] : L.pvel[1 - ppar] + (m - 1) * NC;
+        const float* fo = m == 0 ? L.prho[po] : L.pvel[po] + (m - 1) * NC;
+        ghost_field(fn, fo, m == 0 ? NC : 3 * NC, s_at[lg], (s_grp[lg] >> 11) & 255u, temporal, m == 0 ? 1.0f : 0.0f,
+                    (float*)mac[lg * 8] + m, 8, 4);
     }
-    const int nd = __builtin_popcount(bmask);
-    for (int idx = tid; idx < nd * GREG; idx += 256) {
-        const int d = idx / GREG, r = idx - d * GREG;
-        // the d-th direction of the block's mask
-        uint32_t mm = bmask;
-        for (int skip = 0; skip < d; skip++) mm &= mm - 1u;
-        const int k = __builtin_ctz(mm);
-        const int p = sreg[r];
-        float vn = 0.0f, vo = 0.0f;
-        if (p >= 0) {
-            const float w_k = wk_rt(k);
-            vn = Codec<ST>::load(a.a_new, fidx(p >> 9, k, p & 511), w_k);
-            if (need_old) vo = Codec<ST>::load(a.a_old, fidx(p >> 9, k, p & 511), w_k);
-        }
-        spop[(2 * d) * GREG + r] = vn;
-        spop[(2 * d + 1) * GREG + r] = vo;
-    }
+    if (ddf && tid < ch.n_groups)
+        ghost_field(L.pT[1 - ppar], L.pT[po], NC, s_at[tid], (s_grp[tid] >> 11) & 255u, temporal, 1.0f, mact[tid * 8], 2,
+                    1);
     __syncthreads();
-    const float tc = a.tau_coarse - 0.5f;
-    const float tf = a.tau_fine - 0.5f;
-    float scale = 1.0f;
-    if (tc > 1.0e-6f) {
-        scale = tf / tc;
-        scale = scale > 100.0f ? 100.0f : (scale < 0.01f ? 0.01f : scale);
-    }
-    const int e_end = L.gstart[g + 1];
-    for (int i = L.gstart[g] + tid; i < e_end; i += 256) {
-        const int e0 = a.entries[2 * i];
-        const uint32_t mask = (uint32_t)a.entries[2 * i + 1];
-        const int gb = e0 >> 9, c = e0 & 511;
-        // The fine cell centre lies at (g - 0.5) / 2 in parent cells, g = block
-        // origin (a multiple of 8) + local index + 1, so its fractional part is
-        // 0.25 for an even local index and 0.75 for an odd one (exactly what
-        // (g - 0.5) * 0.5 - floor(...) gives in FP32).  Its corners in the
-        // region: l / 2 and l / 2 + 1, the lower one raised to parent cell 1
-        // at the domain's low faces (region cell 0 is parent cell B / 2).
-        const float wx = (c & 1) ? 0.75f : 0.25f;
-        const float wy = ((c >> 3) & 1) ? 0.75f : 0.25f;
-        const float wz = ((c >> 6) & 1) ? 0.75f : 0.25f;
-        int rlo[3], rhi[3];
-#pragma unroll
-        for (int ax = 0; ax < 3; ax++) {
-            const int l = (c >> (3 * ax)) & 7;
-            const int half = L.borg[(size_t)gb * 3 + ax] / 2;
-            const int lo = half + (l >> 1);
-            rhi[ax] = (l >> 1) + 1;
-            rlo[ax] = (lo < 1 ? 1 : lo) - half;
-        }
-        int rq[8];
-        bool ok[8];
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            rq[q] = ((q & 1) ? rhi[0] : rlo[0]) + 5 * ((q & 2) ? rhi[1] : rlo[1]) + 25 * ((q & 4) ? rhi[2] : rlo[2]);
-            ok[q] = sreg[rq[q]] >= 0;
-        }
-        float v0[8][4], v1[8][4];
-#pragma unroll
-        for (int q = 0; q < 8; q++) {
-            if (ok[q]) {
-                const float rn = smac[0 * GREG + rq[q]], uxn = smac[1 * GREG + rq[q]];
-                const float uyn = smac[2 * GREG + rq[q]], uzn = smac[3 * GREG + rq[q]];
-                const float ro = smac[4 * GREG + rq[q]], uxo = smac[5 * GREG + rq[q]];
-                const float uyo = smac[6 * GREG + rq[q]], uzo = smac[7 * GREG + rq[q]];
-                if (use_old0) {
-                    v0[q][0] = ro * (1.0f - tw0) + rn * tw0;
-                    v0[q][1] = uxo * (1.0f - tw0) + uxn * tw0;
-                    v0[q][2] = uyo * (1.0f - tw0) + uyn * tw0;
-                    v0[q][3] = uzo * (1.0f - tw0) + uzn * tw0;
-                } else {
-                    v0[q][0] = rn; v0[q][1] = uxn; v0[q][2] = uyn; v0[q][3] = uzn;
-                }
-                if (use_old1) {
-                    v1[q][0] = ro * (1.0f - tw1) + rn * tw1;
-                    v1[q][1] = uxo * (1.0f - tw1) + uxn * tw1;
-                    v1[q][2] = uyo * (1.0f - tw1) + uyn * tw1;
-                    v1[q][3] = uzo * (1.0f - tw1) + uzn * tw1;
-                } else {
-                    v1[q][0] = rn; v1[q][1] = uxn; v1[q][2] = uyn; v1[q][3] = uzn;
-                }
-            } else if (q == 0) {
-                v0[0][0] = 1.0f; v0[0][1] = 0.0f; v0[0][2] = 0.0f; v0[0][3] = 0.0f;
-                v1[0][0] = 1.0f; v1[0][1] = 0.0f; v1[0][2] = 0.0f; v1[0][3] = 0.0f;
-            } else {
-#pragma unroll
-                for (int m = 0; m < 4; m++) {
-                    v0[q][m] = v0[0][m];
-                    v1[q][m] = v1[0][m];
-                }
-            }
-        }
-        float r0[4], r1[4];
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            {
-                float c00 = v0[0][m] * (1.0f - wx) + v0[1][m] * wx;
-                float c01 = v0[4][m] * (1.0f - wx) + v0[5][m] * wx;
-                float c10 = v0[2][m] * (1.0f - wx) + v0[3][m] * wx;
-                float c11 = v0[6][m] * (1.0f - wx) + v0[7][m] * wx;
-                float c0 = c00 * (1.0f - wy) + c10 * wy;
-                float c1 = c01 * (1.0f - wy) + c11 * wy;
-                r0[m] = c0 * (1.0f - wz) + c1 * wz;
-            }
-            {
-                float c00 = v1[0][m] * (1.0f - wx) + v1[1][m] * wx;
-                float c01 = v1[4][m] * (1.0f - wx) + v1[5][m] * wx;
-                float c10 = v1[2][m] * (1.0f - wx) + v1[3][m] * wx;
-                float c11 = v1[6][m] * (1.0f - wx) + v1[7][m] * wx;
-                float c0 = c00 * (1.0f - wy) + c10 * wy;
-                float c1 = c01 * (1.0f - wy) + c11 * wy;
-                r1[m] = c0 * (1.0f - wz) + c1 * wz;
-            }
-        }
-#pragma unroll 1
-        for (uint32_t mm = mask; mm != 0u; mm &= mm - 1u) {
-            const int k = __builtin_ctz(mm);
-            const int d = __builtin_popcount(bmask & ((1u << k) - 1u));  // k's slot in the staged region
-            float ln[8], lo[8];
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                ln[q] = spop[(2 * d) * GREG + rq[q]];
-                lo[q] = spop[(2 * d + 1) * GREG + rq[q]];
-            }
-            ghost_blend_store<ST>(a, k, ok, ln, lo, use_old0, use_old1, wx, wy, wz, r0, r1, scale, gb, c);
-        }
+    if (tid >= ch.n_pairs) return;
+    const uint32_t grp = s_grp[pair & 63u];
+    const int gb = L.nb + ch.ghost + (int)(pair >> 19);
+    ghost_store<ST, false>(a, mac, mact, pair, grp, gb, at, vn, vo, temporal, S.comp);
+    if (ddf) {
+        const GhostArgs h = ghost_view(L, par, ppar, temporal, true);
+        ghost_load<ST>(h, at, k, vn, vo);
+        ghost_store<ST, true>(h, mac, mact, pair, grp, gb, at, vn, vo, temporal, S.comp);
     }
 }
 
-// One work-group per work entry: (LevelArgs index, first of 256 ghost
-// entries) for FP32 storage, (LevelArgs index, ghost block) for 16-bit
-// storage.  Thermal populations use the flow's storage.
+// One work-group per chunk; f, and g where the level has it.
 hipError_t ghost_fill(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_chunks, int64_t j,
-                      int storage, int thermal, hipStream_t s) {
+                      int storage, hipStream_t s) {
     if (n_chunks <= 0) return hipSuccess;
     const dim3 grid((unsigned)n_chunks), t(256);
-    const int st = storage;
-    if (st == 1) hipLaunchKernelGGL(ghost_kernel_staged<1>, grid, t, 0, s, las, states, work, j, thermal);
-    else if (st == 2) hipLaunchKernelGGL(ghost_kernel_staged<2>, grid, t, 0, s, las, states, work, j, thermal);
-    else hipLaunchKernelGGL(ghost_kernel<0>, grid, t, 0, s, las, states, work, j, thermal);
+    if (storage == 1) hipLaunchKernelGGL(ghost_kernel<1>, grid, t, 0, s, las, states, work, j);
+    else if (storage == 2) hipLaunchKernelGGL(ghost_kernel<2>, grid, t, 0, s, las, states, work, j);
+    else hipLaunchKernelGGL(ghost_kernel<0>, grid, t, 0, s, las, states, work, j);
     return hipGetLastError();
 }
 
