@@ -80,7 +80,7 @@ struct Level {
     uint8_t* obst = nullptr;
     float* sponge = nullptr;
     float* wall_dist = nullptr;
-    uint8_t* bflags = nullptr;  // per block: any sponge / near-wall / solid cell
+    std::vector<int32_t> wflags;  // per block: WORK_* of its work entry
     int32_t* nbr = nullptr;
     int32_t* borg = nullptr;
     int32_t* order = nullptr;
@@ -657,7 +657,6 @@ int upload_level_args(lb_ctx* c, int li) {
     A.obst = L.obst;
     A.sponge = L.sponge;
     A.wall_dist = L.wall_dist;
-    A.bflags = L.bflags;
     A.nbr = L.nbr;
     A.borg = L.borg;
     A.nb = L.nb;
@@ -814,7 +813,7 @@ int engine_rebuild(lb_engine* e) {
             for (size_t q = 0; q < lev.order_host.size(); q++) {
                 const int32_t b = lev.order_host[q];
                 const bool interior = (int32_t)q < lev.n_int;
-                const lbk::Work w = mkwork(li, b, ci, lev.nbr + (size_t)b * Q, interior ? 0 : lbk::WORK_BOUNDARY);
+                const lbk::Work w = mkwork(li, b, ci, lev.nbr + (size_t)b * Q, lev.wflags[(size_t)b]);
                 (interior ? col : colb).push_back(w);
                 if (ddf) (interior ? tcol : tcolb).push_back(w);
             }
@@ -1267,7 +1266,7 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
     RC(dalloc(c, &L.obst, n4));
     RC(dalloc(c, &L.sponge, n4));
     if (d->wall_dist) RC(dalloc(c, &L.wall_dist, n4));
-    RC(dalloc(c, &L.bflags, (size_t)nb));
+    RC(keep_bytes(c, c->bytes, std::max(nb, 1)));  // (a flag byte per block, now in the work entries)
     RC(dalloc(c, &L.nbr, (size_t)nb * Q));
     RC(dalloc(c, &L.borg, borg.size()));
     RC(dalloc(c, &L.order, (size_t)nb));
@@ -1323,27 +1322,26 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
         }
         RC(h2d(c, L.order, order.data(), order.size()));
         L.order_host = order;
+        L.wflags.assign((size_t)nb, 0);
+        for (int32_t i = 0; i < nb; i++) {
+            const int32_t blk = order[(size_t)i];
+            int32_t f = i < L.n_int ? 0 : lbk::WORK_BOUNDARY;
+            for (size_t k = (size_t)blk * NC; k < (size_t)(blk + 1) * NC; k++) {
+                if (d->sponge[k] > 0.0f) f |= lbk::WORK_SPONGE;
+                if (d->wall_dist && d->wall_dist[k] > 0.0f && d->wall_dist[k] < 10.0f) f |= lbk::WORK_WALL;
+                if (d->obstacle[k]) f |= lbk::WORK_SOLID;
+            }
+            L.wflags[(size_t)blk] = f;
+        }
         std::vector<lbk::Work> wcol((size_t)nb);
         for (int32_t i = 0; i < nb; i++)
             wcol[(size_t)i] = mkwork(L.id - 1, order[(size_t)i], 0, L.nbr + (size_t)order[(size_t)i] * Q,
-                                     i < L.n_int ? 0 : lbk::WORK_BOUNDARY);
+                                     L.wflags[(size_t)order[(size_t)i]]);
         RC(dalloc(c, &L.wcol, wcol.size()));
         RC(h2d(c, L.wcol, wcol.data(), wcol.size()));
         RC(h2d(c, L.obst, d->obstacle, n4));
         RC(h2d(c, L.sponge, d->sponge, n4));
         if (d->wall_dist) RC(h2d(c, L.wall_dist, d->wall_dist, n4));
-        std::vector<uint8_t> bfl((size_t)nb, 0);
-        for (int32_t b = 0; b < nb; b++) {
-            uint8_t f = 0;
-            for (int i = 0; i < NC; i++) {
-                const size_t k = (size_t)b * NC + i;
-                if (d->sponge[k] > 0.0f) f |= 1;
-                if (d->wall_dist && d->wall_dist[k] > 0.0f && d->wall_dist[k] < 10.0f) f |= 2;
-                if (d->obstacle[k]) f |= 4;
-            }
-            bfl[(size_t)b] = f;
-        }
-        RC(h2d(c, L.bflags, bfl.data(), bfl.size()));
     }
     if (ng > 0) {
         std::vector<int32_t> grid(ng);

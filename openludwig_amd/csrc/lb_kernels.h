@@ -94,9 +94,6 @@ struct LevelArgs {
     const uint8_t* obst;
     const float* sponge;
     const float* wall_dist;  // null when the level has no wall distances
-    // per block: bit 0 some cell has sponge > 0; bit 1 some cell has
-    // 0 < wall distance < 10 (the wall model's range); bit 2 some cell is solid
-    const uint8_t* bflags;
     const int32_t* nbr;
     const int32_t* borg;
     int32_t nb;
@@ -120,7 +117,7 @@ struct LevelArgs {
     const uint32_t* ggroup;
     const uint32_t* gpair;
     BouzidiLinks links;
-    int64_t reserved[10];  // the record's size is part of a case's footprint
+    int64_t reserved[11];  // the record's size is part of a case's footprint
 };
 
 // Work list entry.  The neighbour row travels with the entry so that the
@@ -134,8 +131,10 @@ struct Work {
     // stream-collide: the block's neighbour row; ghost fill: the GhostChunk; else null
     const int32_t* nbr_row;
 };
-// some neighbour of the block is neither a block nor a ghost block (domain boundary)
-constexpr int32_t WORK_BOUNDARY = 8;
+// Block flags: some cell has sponge > 0; some cell has 0 < wall distance < 10
+// (the wall model's range); some cell is solid; some neighbour is neither a
+// block nor a ghost block (domain boundary).
+constexpr int32_t WORK_SPONGE = 1, WORK_WALL = 2, WORK_SOLID = 4, WORK_BOUNDARY = 8;
 
 struct ForceArgs {
     // finest level

@@ -62,7 +62,6 @@ struct CollideArgs {
     const uint8_t* obst;
     const float* sponge;
     const float* wall_dist;
-    const uint8_t* bflags;
     const int32_t* nbr;
     const int32_t* borg;
     int32_t nb;
@@ -161,7 +160,6 @@ __device__ __forceinline__ CollideArgs collide_view(const LevelArgs& L, const Ca
     a.obst = L.obst;
     a.sponge = L.sponge;
     a.wall_dist = L.wall_dist;
-    a.bflags = L.bflags;
     a.nbr = L.nbr;
     a.borg = L.borg;
     a.nb = L.nb;
@@ -719,7 +717,7 @@ struct CollideLds {
 
 template <int ST, class OffT, bool BND>
 __device__ __forceinline__ void collide_body(const CollideArgs& a, CollideLds<ST, OffT>& lds, int b, int half,
-                                             int tid) {
+                                             int flags, int tid) {
     constexpr int ESZ = ST == 0 ? 4 : 2;
     constexpr int ROWS = OUT_ROWS<ST>;
     // opaque to the boundary instance, so that nothing the two instances share
@@ -732,14 +730,24 @@ __device__ __forceinline__ void collide_body(const CollideArgs& a, CollideLds<ST
     const int x = c & 7, y = (c >> 3) & 7;
     const int wv = tid >> 6;
     const size_t i4 = (size_t)b * NC + c;
-    bool is_obs = false;
-    if constexpr (ST != 0) is_obs = __builtin_nontemporal_load(&gp(a.obst)[i4]) != 0;
 
     // STEP 1: pull (kernel_cumulant.jl:86-168).  All 27 loads are issued
     // before any is used, each one table read and one add.
     const int oxp = x == 0 ? -1 : 0, oxm = x == 7 ? 1 : 0;
     const int oyp = y == 0 ? -1 : 0, oym = y == 7 ? 1 : 0;
     const OffT cb = (OffT)c * (OffT)ESZ;
+    // Single-use inputs: non-temporal loads keep L2 for the neighbour pulls.
+    // A block with no solid, sponge or near-wall cell skips them (the values
+    // they would give: not solid, sponge 0, no wall model), 9 of 141 bytes a
+    // cell in 16-bit storage.  Its flags come with the work entry, so the
+    // branches wait for nothing and can stand before the pull; as a byte loaded
+    // per block the flags cost the 16-bit forms more than the loads.  Coarse
+    // step: FP16 cube (11.4 M cells) 2.52 -> 2.38 ms, thermal wing (10.7 M)
+    // 4.56 -> 4.46 ms, FP32 unchanged.
+    const bool is_obs = (flags & WORK_SOLID) ? __builtin_nontemporal_load(&gp(a.obst)[i4]) != 0 : false;
+    const float sp = (flags & WORK_SPONGE) ? __builtin_nontemporal_load(&gp(a.sponge)[i4]) : 0.0f;
+    const float wdist =
+        (a.wall_model == 1 && (flags & WORK_WALL)) ? __builtin_nontemporal_load(&gp(a.wall_dist)[i4]) : 0.0f;
     const VelTile vtl = vel_tile_load<OffT>(a.vel_in, vtab, half, c, tid);
     Pulled<ST> P[27];
     pull<ST, OffT>(a.f_in, ptab + wv * 27, cb, oxp, oxm, oyp, oym, P);
@@ -755,21 +763,6 @@ __device__ __forceinline__ void collide_body(const CollideArgs& a, CollideLds<ST
 #pragma unroll
         for (int d = 0; d < 3; d++) VN[n][d] = vt[vt_index(d, wv + dz, y + dy, x + dx)];
     }
-    // single-use inputs: non-temporal loads keep L2 for the neighbour pulls
-    // FP32: a block with no solid, sponge or near-wall cell skips those loads
-    // (the values they would give: not solid, sponge 0, no wall model); the
-    // branch comes after the pull and stencil loads so that it does not hold
-    // them back.  Measured on the cube case: FP32 finest collide -2 %; the
-    // 16-bit forms, limited by loads in flight rather than bytes, lose 1.4 to
-    // 2.3 % to the extra branch and keep the unconditional loads (bfl = 7).
-    uint32_t bfl = 7u;
-    if constexpr (ST == 0) {
-        bfl = gp(a.bflags)[b];
-        is_obs = (bfl & 4u) ? __builtin_nontemporal_load(&gp(a.obst)[i4]) != 0 : false;
-    }
-    const float sp = (bfl & 1u) ? __builtin_nontemporal_load(&gp(a.sponge)[i4]) : 0.0f;
-    const float wdist =
-        (a.wall_model == 1 && (bfl & 2u)) ? __builtin_nontemporal_load(&gp(a.wall_dist)[i4]) : 0.0f;
     uint32_t empty = 0u;
     if constexpr (BND)
         empty = pull_mirrors<ST, OffT>(a.f_in, wave_miss(lds.smask, wv), (OffT)b * (OffT)(Q * NC * ESZ) + cb, oxp, oxm,
@@ -1114,9 +1107,9 @@ __device__ __forceinline__ void collide_tile(const LevelArgs* __restrict__ las, 
     if (!live(L, S, j)) return;
     const CollideArgs a = collide_view(L, S, j);
     if (wk.flags & WORK_BOUNDARY)
-        collide_body<ST, OffT, true>(a, lds, b, half, tid);
+        collide_body<ST, OffT, true>(a, lds, b, half, wk.flags, tid);
     else
-        collide_body<ST, OffT, false>(a, lds, b, half, tid);
+        collide_body<ST, OffT, false>(a, lds, b, half, wk.flags, tid);
 }
 
 template <int ST, class OffT, int W>
@@ -1212,7 +1205,7 @@ struct ThermalLds {
 
 template <int ST, class OffT, bool BND>
 __device__ __forceinline__ void thermal_body(const ThermalArgs& a, ThermalLds<ST, OffT>& lds, int b, int half,
-                                             int tid) {
+                                             int flags, int tid) {
     constexpr int ESZ = ST == 0 ? 4 : 2;
     if constexpr (BND) asm volatile("" : "+v"(tid));  // as in collide_body
     const int c = (half << 8) | tid;
@@ -1227,7 +1220,8 @@ __device__ __forceinline__ void thermal_body(const ThermalArgs& a, ThermalLds<ST
     const OffT cb = (OffT)c * (OffT)ESZ;
     Pulled<ST> P[27];
     pull<ST, OffT>(a.g_in, ptab + wv * 27, cb, oxp, oxm, oyp, oym, P);
-    const bool is_obs = gp(a.obst)[i4] != 0;
+    const bool is_obs = (flags & WORK_SOLID) ? gp(a.obst)[i4] != 0 : false;
+    const float sponge = (flags & WORK_SPONGE) ? gp(a.sponge)[i4] : 0.0f;
     uint32_t empty = 0u;
     if constexpr (BND)
         empty = pull_mirrors<ST, OffT>(a.g_in, wave_miss(lds.smask, wv), (OffT)b * (OffT)(Q * NC * ESZ) + cb, oxp, oxm,
@@ -1265,7 +1259,7 @@ __device__ __forceinline__ void thermal_body(const ThermalArgs& a, ThermalLds<ST
         if (a.store_T) a.T_out[i4] = a.adiabatic == 1 ? Tsum : a.T_wall;
     } else {
         float Tl = fmaxf(Tsum, 0.01f);
-        const float sp = a.sponge[i4];
+        const float sp = sponge;
         if (sp > 0.0f) {
             Tl = Tl * (1.0f - sp) + a.T_inlet * sp;
             ux = ux * (1.0f - sp) + a.u_inlet * sp;
@@ -1289,7 +1283,7 @@ __device__ __forceinline__ void thermal_body(const ThermalArgs& a, ThermalLds<ST
 }
 
 template <int ST, class OffT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ST == 0 ? 5 : 7)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ST == 0 ? 5 : 6)))
 thermal_kernel(const LevelArgs* __restrict__ las, const CaseState* __restrict__ states,
                const Work* __restrict__ work, int32_t n_tiles, int64_t j, int32_t sched) {
     __shared__ ThermalLds<ST, OffT> lds;
@@ -1303,9 +1297,9 @@ thermal_kernel(const LevelArgs* __restrict__ las, const CaseState* __restrict__ 
     if (!live(L, S, j)) return;
     const ThermalArgs a = thermal_view(L, S, j);
     if (wk.flags & WORK_BOUNDARY)
-        thermal_body<ST, OffT, true>(a, lds, wk.item, half, (int)threadIdx.x);
+        thermal_body<ST, OffT, true>(a, lds, wk.item, half, wk.flags, (int)threadIdx.x);
     else
-        thermal_body<ST, OffT, false>(a, lds, wk.item, half, (int)threadIdx.x);
+        thermal_body<ST, OffT, false>(a, lds, wk.item, half, wk.flags, (int)threadIdx.x);
 }
 
 template <int ST>
