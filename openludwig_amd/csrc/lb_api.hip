@@ -55,7 +55,7 @@ struct Kern {
     hipError_t (*forces)(const lbk::ForceArgs&, int, double*, hipStream_t);
     hipError_t (*stats)(const void*, const float*, const float*, const uint8_t*, int32_t, int, double*, int,
                         hipStream_t);
-    hipError_t (*finite_count)(const lbk::FiniteEntry*, int32_t, int32_t, int32_t*, hipStream_t);
+    hipError_t (*finite_count)(const lbk::FiniteEntry*, int32_t, int64_t, int32_t*, hipStream_t);
     hipError_t (*engine_forces)(const lbk::EngineForce*, const lbk::CaseState*, const lbk::Work*, int32_t,
                                 const int32_t*, int32_t, int64_t, hipStream_t);
 };
@@ -878,7 +878,11 @@ hipError_t engine_issue_step(lb_engine* e) {
 
 // Divergence check entry of one level: its density and velocity in buffer
 // `cur` (the output of the last completed coarse step).
-constexpr int32_t kFiniteGroups = 64;  // work-groups per (case, level) entry
+int64_t largest(const std::vector<lbk::FiniteEntry>& ents) {  // cells of the largest entry
+    int64_t n = 0;
+    for (const lbk::FiniteEntry& e : ents) n = std::max(n, e.n);
+    return n;
+}
 lbk::FiniteEntry finite_entry(const Level& L, int cur, int32_t slot) {
     lbk::FiniteEntry e;
     e.rho = L.rho[cur];
@@ -1684,7 +1688,7 @@ int lb_check_finite(lb_ctx* c, int64_t* n_nonfinite) {
         HIPCHK(c, hipMemcpyAsync(c->fin_ents, ents.data(), ents.size() * sizeof(lbk::FiniteEntry),
                                  hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipMemsetAsync(c->fin_count, 0, sizeof(int32_t), c->stream));
-        HIPCHK(c, c->k->finite_count(c->fin_ents, (int32_t)ents.size(), kFiniteGroups, c->fin_count, c->stream));
+        HIPCHK(c, c->k->finite_count(c->fin_ents, (int32_t)ents.size(), largest(ents), c->fin_count, c->stream));
         HIPCHK(c, hipMemcpyAsync(&count, c->fin_count, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
     }
@@ -1953,7 +1957,7 @@ int lb_engine_check_finite(lb_engine* e, lb_ctx** diverged, int32_t cap, int32_t
     EHIPCHK(e, hipMemcpyAsync(e->fin_ents, ents.data(), ents.size() * sizeof(lbk::FiniteEntry), hipMemcpyHostToDevice,
                               e->stream));
     EHIPCHK(e, hipMemsetAsync(e->fin_counts, 0, nc * sizeof(int32_t), e->stream));
-    EHIPCHK(e, e->k->finite_count(e->fin_ents, (int32_t)ents.size(), kFiniteGroups, e->fin_counts, e->stream));
+    EHIPCHK(e, e->k->finite_count(e->fin_ents, (int32_t)ents.size(), largest(ents), e->fin_counts, e->stream));
     EHIPCHK(e, hipMemcpyAsync(counts.data(), e->fin_counts, nc * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
     EHIPCHK(e, hipStreamSynchronize(e->stream));
     int32_t n = 0;

@@ -216,8 +216,8 @@ struct FiniteEntry {
     hipError_t forces(const lbk::ForceArgs& a, int n_groups, double* out9, hipStream_t s);               \
     hipError_t stats(const void* f, const float* rho, const float* vel, const uint8_t* obst, int32_t nb,  \
                      int storage, double* partials, int n_groups, hipStream_t s);                        \
-    hipError_t finite_count(const lbk::FiniteEntry* ents, int32_t n_ents, int32_t groups_per_entry,          \
-                            int32_t* counts, hipStream_t s);                                             \
+    hipError_t finite_count(const lbk::FiniteEntry* ents, int32_t n_ents, int64_t largest, int32_t* counts, \
+                            hipStream_t s);                                                              \
     hipError_t engine_forces(const lbk::EngineForce* recs, const lbk::CaseState* states, const lbk::Work* work,  \
                              int32_t n_chunks, const int32_t* rec_idx, int32_t n_recs, int64_t j, hipStream_t s); \
     }

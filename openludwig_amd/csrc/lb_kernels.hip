@@ -744,7 +744,7 @@ __device__ __forceinline__ void collide_body(const CollideArgs& a, CollideLds<ST
     // per block the flags cost the 16-bit forms more than the loads.  Coarse
     // step: FP16 cube (11.4 M cells) 2.52 -> 2.38 ms, thermal wing (10.7 M)
     // 4.56 -> 4.46 ms, FP32 unchanged.
-    const bool is_obs = (flags & WORK_SOLID) ? __builtin_nontemporal_load(&gp(a.obst)[i4]) != 0 : false;
+    const uint32_t solid = (flags & WORK_SOLID) ? __builtin_nontemporal_load(&gp(a.obst)[i4]) : 0u;
     const float sp = (flags & WORK_SPONGE) ? __builtin_nontemporal_load(&gp(a.sponge)[i4]) : 0.0f;
     const float wdist =
         (a.wall_model == 1 && (flags & WORK_WALL)) ? __builtin_nontemporal_load(&gp(a.wall_dist)[i4]) : 0.0f;
@@ -799,6 +799,7 @@ __device__ __forceinline__ void collide_body(const CollideArgs& a, CollideLds<ST
         if (cz == -1) jz += -val;
     }
 
+    const bool is_obs = solid != 0u;
     void* const fo = a.f_out;
     GF* __restrict__ vo = gp(a.vel_out);
     GF* __restrict__ ro = gp(a.rho_out);
@@ -1801,17 +1802,32 @@ __device__ bool trilinear_sample(const ForceArgs& a, float px, float py, float p
 // fallback's side test, the wall distance and the stress (each a sign flip,
 // exact), so the maps are computed here with n -> -n; the integrated sums
 // are then not used.
-// One work-group: triangles chunk*256 .. chunk*256+255, partial sums into
-// a.partials[chunk].
+// One work-group: triangles chunk*256 .. chunk*256+255, a work-item each, and
+// FORCE_THREADS work-items for the search; partial sums into a.partials[chunk].
+constexpr int FORCE_THREADS = 1024;
+struct SearchTri {
+    float x, y, z, nx, ny, nz;
+};
+struct SearchHit {
+    int blk, c;  // the cell found, or blk = -1
+    float dn;    // its distance along the normal
+};
 __device__ void forces_block(const ForceArgs& a, int64_t chunk) {
     __shared__ double red[9][256];
-    int64_t i = chunk * 256 + threadIdx.x;
+    __shared__ SearchTri left[256];
+    __shared__ SearchHit hits[256];
+    __shared__ int n_left;
+    const int tid = (int)threadIdx.x;
+    int64_t i = chunk * 256 + tid;
     float d9[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    if (i < a.n_tri) {
-        float tx = a.cx[i] + a.off_x, ty = a.cy[i] + a.off_y, tz = a.cz[i] + a.off_z;
-        float n_x = a.side * a.nx[i], n_y = a.side * a.ny[i], n_z = a.side * a.nz[i];
-        float brho = 1.0f, bux = 0.0f, buy = 0.0f, buz = 0.0f, bwd = 1.0f, bq = 0.0f;
-        bool found = false;
+    const bool mine = tid < 256 && i < a.n_tri;
+    int slot = 0;
+    float tx = 0.0f, ty = 0.0f, tz = 0.0f, n_x = 0.0f, n_y = 0.0f, n_z = 0.0f;
+    float brho = 1.0f, bux = 0.0f, buy = 0.0f, buz = 0.0f, bwd = 1.0f, bq = 0.0f;
+    bool found = false;
+    if (mine) {
+        tx = a.cx[i] + a.off_x, ty = a.cy[i] + a.off_y, tz = a.cz[i] + a.off_z;
+        n_x = a.side * a.nx[i], n_y = a.side * a.ny[i], n_z = a.side * a.nz[i];
         for (int pi = 1; pi <= a.search_radius; pi++) {
             float dc = (float)pi + 0.5f;
             float px = tx + n_x * dc * a.dx, py = ty + n_y * dc * a.dx, pz = tz + n_z * dc * a.dx;
@@ -1824,39 +1840,95 @@ __device__ void forces_block(const ForceArgs& a, int64_t chunk) {
                 brho = r; bux = u; buy = v; buz = w; bwd = dc; bq = wq; found = true;
             }
         }
-        if (!found) {
-            float gxf = tx / a.dx, gyf = ty / a.dx, gzf = tz / a.dx;
-            int g_x = (int)floorf(gxf) + 1, g_y = (int)floorf(gyf) + 1, g_z = (int)floorf(gzf) + 1;
-            float best = 1e10f;
-            for (int rad = 1; rad <= a.search_radius; rad++) {
-                if (found) break;
-                for (int dz = -rad; dz <= rad; dz++)
-                    for (int dy = -rad; dy <= rad; dy++)
-                        for (int ddx = -rad; ddx <= rad; ddx++) {
-                            bool shell = (abs(ddx) == rad) || (abs(dy) == rad) || (abs(dz) == rad);
-                            if (!shell) continue;
-                            int cgx = g_x + ddx, cgy = g_y + dy, cgz = g_z + dz;
-                            int blk, c;
-                            if (!cell_at(a, cgx, cgy, cgz, blk, c)) continue;
-                            size_t i4 = (size_t)blk * NC + c;
-                            if (a.obst[i4]) continue;
-                            float ccx = ((float)cgx - 0.5f) * a.dx, ccy = ((float)cgy - 0.5f) * a.dx,
-                                  ccz = ((float)cgz - 0.5f) * a.dx;
-                            float dxp = ccx - tx, dyp = ccy - ty, dzp = ccz - tz;
-                            float dn = dxp * n_x + dyp * n_y + dzp * n_z;
-                            if (dn <= 0.0f) continue;
-                            float dsq = dxp * dxp + dyp * dyp + dzp * dzp;
-                            if (dsq < best) {
-                                size_t iv = (size_t)blk * 3 * NC + c;
-                                best = dsq;
-                                brho = a.rho[i4];
-                                bux = a.vel[iv]; buy = a.vel[iv + NC]; buz = a.vel[iv + 2 * NC];
-                                bwd = dn / a.dx;
-                                found = true;
-                            }
-                        }
+    }
+    // Triangles whose probes met no fluid: the nearest fluid cell on the
+    // normal's side, in the first shell of cells around the triangle that has
+    // one (the first such cell in the reference's loop order).  The work-group
+    // lists them and searches each with 16 lanes, one sweep over all shells, a
+    // lane per row of cells with 8 solid flags in one load.  Bound by latency: one work-item per triangle
+    // walking 11^3 cells, each a block lookup and then a flag, held less than
+    // one wave per SIMD for 509 us on the 40,400-triangle wing (400 such
+    // triangles outside, 28,300 inside); now 152 us on average of the two sides,
+    // 15 us as before where no triangle needs it.
+    if (tid == 0) n_left = 0;
+    __syncthreads();
+    if (mine && !found) {
+        const int at = atomicAdd(&n_left, 1);
+        left[at] = {tx, ty, tz, n_x, n_y, n_z};
+        slot = at;
+    }
+    __syncthreads();
+    const int sub = tid & 15;
+    for (int t = tid >> 4; t < n_left; t += FORCE_THREADS / 16) {
+        const SearchTri q = left[t];
+        float gxf = q.x / a.dx, gyf = q.y / a.dx, gzf = q.z / a.dx;
+        int g_x = (int)floorf(gxf) + 1, g_y = (int)floorf(gyf) + 1, g_z = (int)floorf(gzf) + 1;
+        const int R = a.search_radius, side = 2 * R + 1;
+        uint64_t key = ~0ull;  // shell, then squared distance
+        int64_t place = INT64_MAX;
+        SearchHit hit{-1, 0, 0.0f};
+        const int x0 = max(g_x - R, 1), x1 = min(g_x + R, a.gdx * BS);
+        for (int row = sub; row < side * side; row += 16) {
+            const int dy = row % side - R, dz = row / side - R;
+            const int cgy = g_y + dy, cgz = g_z + dz;
+            if (cgy < 1 || cgz < 1 || cgy > a.gdy * BS || cgz > a.gdz * BS) continue;
+            const int32_t* grid = a.grid + (size_t)a.gdx * ((size_t)((cgy - 1) >> 3) + (size_t)a.gdy * ((cgz - 1) >> 3));
+            const int line = ((cgy - 1) & 7) * BS + ((cgz - 1) & 7) * BS * BS;
+            const float ccy = ((float)cgy - 0.5f) * a.dx, ccz = ((float)cgz - 0.5f) * a.dx;
+            const float dyp = ccy - q.y, dzp = ccz - q.z;
+            // the row's cells of up to three blocks at a time, 8 flags in one load each
+            for (int bx0 = (x0 - 1) >> 3; bx0 <= (x1 - 1) >> 3; bx0 += 3) {
+                int id[3];
+                uint64_t flags[3];
+#pragma unroll
+                for (int u = 0; u < 3; u++) id[u] = bx0 + u <= (x1 - 1) >> 3 ? grid[bx0 + u] : -1;
+#pragma unroll
+                for (int u = 0; u < 3; u++)
+                    flags[u] = id[u] >= 0 ? *(const uint64_t*)(a.obst + (size_t)id[u] * NC + line) : ~0ull;
+#pragma unroll
+                for (int u = 0; u < 3; u++) {
+                    // bit 8 l + 7 set for each fluid cell l (a zero byte)
+                    const uint64_t low = 0x7f7f7f7f7f7f7f7full;
+                    uint64_t fluid = ~(((flags[u] & low) + low) | flags[u] | low);
+                    for (; fluid != 0; fluid &= fluid - 1) {
+                        const int lx = __builtin_ctzll(fluid) >> 3, cgx = (bx0 + u) * BS + lx + 1;
+                        const int ddx = cgx - g_x;
+                        if (cgx < x0 || cgx > x1) continue;
+                        const int rad = max(abs(ddx), max(abs(dy), abs(dz)));
+                        const float ccx = ((float)cgx - 0.5f) * a.dx;
+                        const float dxp = ccx - q.x;
+                        const float dn = dxp * q.nx + dyp * q.ny + dzp * q.nz;
+                        const float dsq = dxp * dxp + dyp * dyp + dzp * dzp;
+                        const uint64_t k = (uint64_t)(uint32_t)rad << 32 | __float_as_uint(dsq);
+                        // a lane meets its cells in loop order: an equal key does not replace
+                        if (rad > 0 && !(dn <= 0.0f) && dsq < 1e10f && k < key)
+                            key = k, place = (int64_t)row * side + ddx + R, hit = {id[u], line + lx, dn};
+                    }
+                }
             }
         }
+        // the least (shell, distance, place) of the 16 lanes
+        uint64_t lk = key;
+        int64_t lp = place;
+        for (int off = 8; off > 0; off >>= 1) {
+            const uint64_t ok = (uint64_t)__shfl_xor((unsigned long long)lk, off, 16);
+            const int64_t op = (int64_t)__shfl_xor((long long)lp, off, 16);
+            if (ok < lk || (ok == lk && op < lp)) lk = ok, lp = op;
+        }
+        if (key == lk && place == lp && (sub == 0 || lk != ~0ull)) hits[t] = hit;
+    }
+    __syncthreads();
+    if (mine && !found) {
+        const SearchHit h = hits[slot];
+        if (h.blk >= 0) {
+            const size_t i4 = (size_t)h.blk * NC + h.c, iv = (size_t)h.blk * 3 * NC + h.c;
+            brho = a.rho[i4];
+            bux = a.vel[iv]; buy = a.vel[iv + NC]; buz = a.vel[iv + 2 * NC];
+            bwd = h.dn / a.dx;
+            found = true;
+        }
+    }
+    if (mine) {
         float p = 0.0f, tx_ = 0.0f, ty_ = 0.0f, tz_ = 0.0f;
         if (found) {
             // compute_stress_from_cell (surface.jl:143-190)
@@ -1897,24 +1969,26 @@ __device__ void forces_block(const ForceArgs& a, int64_t chunk) {
         d9[7] = rz * dFx - rx * dFz;
         d9[8] = rx * dFy - ry * dFx;
     }
+    if (tid < 256) {
 #pragma unroll
-    for (int j = 0; j < 9; j++) red[j][threadIdx.x] = (double)d9[j];
+        for (int j = 0; j < 9; j++) red[j][tid] = (double)d9[j];
+    }
     __syncthreads();
     for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s)
+        if (tid < s)
 #pragma unroll
-            for (int j = 0; j < 9; j++) red[j][threadIdx.x] += red[j][threadIdx.x + s];
+            for (int j = 0; j < 9; j++) red[j][tid] += red[j][tid + s];
         __syncthreads();
     }
-    if (threadIdx.x < 9) a.partials[(size_t)chunk * 9 + threadIdx.x] = red[threadIdx.x][0];
+    if (tid < 9) a.partials[(size_t)chunk * 9 + tid] = red[tid][0];
 }
 
-__global__ void __launch_bounds__(256) forces_kernel(const ForceArgs a) { forces_block(a, blockIdx.x); }
+__global__ void __launch_bounds__(FORCE_THREADS) forces_kernel(const ForceArgs a) { forces_block(a, blockIdx.x); }
 
 hipError_t forces(const ForceArgs& a, int n_groups, double* out9, hipStream_t s) {
     (void)out9;
     if (a.n_tri <= 0) return hipSuccess;
-    hipLaunchKernelGGL(forces_kernel, dim3((unsigned)n_groups), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(forces_kernel, dim3((unsigned)n_groups), dim3(FORCE_THREADS), 0, s, a);
     return hipGetLastError();
 }
 
@@ -1932,7 +2006,7 @@ __device__ __forceinline__ bool sample_step(const EngineForce& R, const CaseStat
     return S.active && t <= S.n_total && t > R.ramp && (t % R.diag) == 0;
 }
 
-__global__ void __launch_bounds__(256) engine_forces_kernel(const EngineForce* __restrict__ recs,
+__global__ void __launch_bounds__(FORCE_THREADS) engine_forces_kernel(const EngineForce* __restrict__ recs,
                                                             const CaseState* __restrict__ states,
                                                             const Work* __restrict__ work, int64_t j) {
     const Work wk = work[blockIdx.x];
@@ -1945,26 +2019,28 @@ __global__ void __launch_bounds__(256) engine_forces_kernel(const EngineForce* _
     forces_block(a, wk.item);
 }
 
+// One work-group per record, a work-item per component (each component's sum
+// runs in chunk order).
 __global__ void engine_forces_reduce(const EngineForce* __restrict__ recs, const CaseState* __restrict__ states,
-                                     const int32_t* __restrict__ rec_idx, int32_t n, int64_t j) {
-    const int32_t q = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (q >= n) return;
-    const EngineForce& R = recs[rec_idx[q]];
+                                     const int32_t* __restrict__ rec_idx, int64_t j) {
+    const EngineForce& R = recs[rec_idx[blockIdx.x]];
     int64_t t;
     if (!sample_step(R, states[R.ci], j, &t)) return;
-    double s9[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    for (int32_t g = 0; g < R.n_groups; g++)
-        for (int c = 0; c < 9; c++) s9[c] += R.a.partials[(size_t)g * 9 + c];
-    for (int c = 0; c < 9; c++) R.acc[c] += s9[c];
-    R.acc[9] += 1.0;
+    const int c = (int)threadIdx.x;
+    if (c < 9) {
+        double sum = 0.0;
+        for (int32_t g = 0; g < R.n_groups; g++) sum += R.a.partials[(size_t)g * 9 + c];
+        R.acc[c] += sum;
+    } else if (c == 9) {
+        R.acc[9] += 1.0;
+    }
 }
 
 hipError_t engine_forces(const EngineForce* recs, const CaseState* states, const Work* work, int32_t n_chunks,
                          const int32_t* rec_idx, int32_t n_recs, int64_t j, hipStream_t s) {
     if (n_chunks <= 0 || n_recs <= 0) return hipSuccess;
-    hipLaunchKernelGGL(engine_forces_kernel, dim3((unsigned)n_chunks), dim3(256), 0, s, recs, states, work, j);
-    hipLaunchKernelGGL(engine_forces_reduce, dim3((unsigned)((n_recs + 63) / 64)), dim3(64), 0, s, recs, states,
-                       rec_idx, n_recs, j);
+    hipLaunchKernelGGL(engine_forces_kernel, dim3((unsigned)n_chunks), dim3(FORCE_THREADS), 0, s, recs, states, work, j);
+    hipLaunchKernelGGL(engine_forces_reduce, dim3((unsigned)n_recs), dim3(64), 0, s, recs, states, rec_idx, j);
     return hipGetLastError();
 }
 
@@ -2035,24 +2111,40 @@ hipError_t stats(const void* f, const float* rho, const float* vel, const uint8_
 // ---------------------------------------------------------------------------
 // Divergence check: non-finite density and velocity values per case.  Row y
 // of the grid is one (case, level) entry; its work-groups stride over the
-// entry's n cells (rho) and 3n velocity components and add their count to
-// counts[entry.slot].
+// entry's n cells (rho) and 3n velocity components (n a multiple of 512) in
+// 16-byte loads, four in flight, and add their count to counts[entry.slot].
+// A plain stream, so the work-groups follow the largest entry: with 64 per
+// entry and 4-byte loads it ran at 0.3 TB/s (221 us at 4.5 M cells, 3.36 ms at
+// 52.5 M), now 16 us and 0.18 ms with the call.
 __global__ void __launch_bounds__(256) finite_kernel(const FiniteEntry* __restrict__ ents, int32_t* counts) {
     const FiniteEntry e = ents[blockIdx.y];
+    const int64_t nr = e.n / 4, n = 4 * nr, stride = (int64_t)gridDim.x * 256;
+    const GV4U* rho = (const GV4U*)e.rho;
+    const GV4U* vel = (const GV4U*)e.vel;
     int32_t bad = 0;
-    const int64_t stride = (int64_t)gridDim.x * 256;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < e.n; i += stride) bad += isfinite(e.rho[i]) ? 0 : 1;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < 3 * e.n; i += stride)
-        bad += isfinite(e.vel[i]) ? 0 : 1;
+    auto count = [](v4u v) {
+        int32_t k = 0;
+#pragma unroll
+        for (int m = 0; m < 4; m++) k += (v[m] & 0x7f800000u) == 0x7f800000u ? 1 : 0;
+        return k;
+    };
+    auto at = [&](int64_t i) { return i < nr ? rho[i] : vel[i - nr]; };
+    int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    for (; i + 3 * stride < n; i += 4 * stride) {
+        const v4u v0 = at(i), v1 = at(i + stride), v2 = at(i + 2 * stride), v3 = at(i + 3 * stride);
+        bad += count(v0) + count(v1) + count(v2) + count(v3);
+    }
+    for (; i < n; i += stride) bad += count(at(i));
     for (int off = 32; off > 0; off >>= 1) bad += __shfl_down(bad, off, 64);
     if ((threadIdx.x & 63) == 0 && bad != 0) atomicAdd(&counts[e.slot], bad);
 }
 
-hipError_t finite_count(const FiniteEntry* ents, int32_t n_ents, int32_t groups_per_entry, int32_t* counts,
-                        hipStream_t s) {
+hipError_t finite_count(const FiniteEntry* ents, int32_t n_ents, int64_t largest, int32_t* counts, hipStream_t s) {
     if (n_ents <= 0) return hipSuccess;
-    hipLaunchKernelGGL(finite_kernel, dim3((unsigned)groups_per_entry, (unsigned)n_ents), dim3(256), 0, s, ents,
-                       counts);
+    // 16 bytes per work-item and pass, 4 passes in flight, up to 8 work-groups per CU
+    const int64_t want = (largest + 1023) / 1024;
+    const unsigned groups = (unsigned)(want < 8 ? 8 : (want > 2048 ? 2048 : want));
+    hipLaunchKernelGGL(finite_kernel, dim3(groups, (unsigned)n_ents), dim3(256), 0, s, ents, counts);
     return hipGetLastError();
 }
 
