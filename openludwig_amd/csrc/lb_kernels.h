@@ -216,6 +216,8 @@ struct FiniteEntry {
     hipError_t forces(const lbk::ForceArgs& a, int n_groups, double* out9, hipStream_t s);               \
     hipError_t stats(const void* f, const float* rho, const float* vel, const uint8_t* obst, int32_t nb,  \
                      int storage, double* partials, int n_groups, hipStream_t s);                        \
+    hipError_t export_rows(const void* src, const int32_t* inv, int32_t nb, int32_t n_comp, int storage,    \
+                           int64_t row0, int32_t n_rows, float* out, hipStream_t s);                     \
     hipError_t finite_count(const lbk::FiniteEntry* ents, int32_t n_ents, int64_t largest, int32_t* counts, \
                             hipStream_t s);                                                              \
     hipError_t engine_forces(const lbk::EngineForce* recs, const lbk::CaseState* states, const lbk::Work* work,  \

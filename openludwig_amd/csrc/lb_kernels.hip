@@ -2109,6 +2109,43 @@ hipError_t stats(const void* f, const float* rho, const float* vel, const uint8_
 }
 
 // ---------------------------------------------------------------------------
+// Rows row0 .. row0 + n_rows - 1 of a field in the caller's layout, FP32: row
+// k nb + i holds component k of the caller's block i (512 cells).  The blocks
+// are put in the caller's order and 16-bit populations decoded here, so that
+// the host copies what arrives as it is.  out is pinned host memory, written
+// over the link in whole 1 KiB waves; two rows per work-group.
+template <int ST>
+__global__ void __launch_bounds__(256) export_kernel(const void* __restrict__ src, const int32_t* __restrict__ inv,
+                                                     int32_t nb, int32_t n_comp, int64_t row0, int32_t n_rows,
+                                                     float* __restrict__ out) {
+    const int32_t r = (int32_t)blockIdx.x * 2 + (int32_t)(threadIdx.x >> 7);
+    if (r >= n_rows) return;
+    const int32_t k = (int32_t)((row0 + r) / nb), i = (int32_t)((row0 + r) - (int64_t)k * nb);
+    const int c = 4 * (int)(threadIdx.x & 127);
+    const size_t at = ((size_t)inv[i] * (size_t)n_comp + (size_t)k) * NC + (size_t)c;
+    const float w = wk_rt(k);
+    v4u v;
+    if constexpr (ST == 0) {
+        v = *(const GV4U*)((const GF*)src + at);
+    } else {
+        typedef uint16_t v4h __attribute__((ext_vector_type(4)));
+        const v4h h = *(const __attribute__((address_space(1))) v4h*)((const GU16*)src + at);
+#pragma unroll
+        for (int m = 0; m < 4; m++) v[m] = __float_as_uint(Codec<ST>::value(h[m], w));
+    }
+    __builtin_nontemporal_store(v, (GV4U*)((GF*)out + (size_t)r * NC + c));
+}
+hipError_t export_rows(const void* src, const int32_t* inv, int32_t nb, int32_t n_comp, int storage, int64_t row0,
+                       int32_t n_rows, float* out, hipStream_t s) {
+    if (n_rows <= 0) return hipSuccess;
+    const dim3 grid((unsigned)((n_rows + 1) / 2)), t(256);
+    if (storage == 1) hipLaunchKernelGGL(export_kernel<1>, grid, t, 0, s, src, inv, nb, n_comp, row0, n_rows, out);
+    else if (storage == 2) hipLaunchKernelGGL(export_kernel<2>, grid, t, 0, s, src, inv, nb, n_comp, row0, n_rows, out);
+    else hipLaunchKernelGGL(export_kernel<0>, grid, t, 0, s, src, inv, nb, n_comp, row0, n_rows, out);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // Divergence check: non-finite density and velocity values per case.  Row y
 // of the grid is one (case, level) entry; its work-groups stride over the
 // entry's n cells (rho) and 3n velocity components (n a multiple of 512) in
