@@ -1336,10 +1336,10 @@ hipError_t thermal(const LevelArgs* las, const CaseState* states, const Work* wo
 // density and velocity blends of the chunk's groups into LDS, a work-item per
 // (group, field), then a work-item per (group, direction).  Against a
 // work-item per ghost cell (FP32) and per-block staging of the 5^3 parent
-// region in LDS (16-bit), one launch of the finest fill: 22.8 -> 16.0 us (FP32
-// sphere, 500 chunks), 44.5 -> 34.4 us (6.1 M-cell cube), 142 -> 123 us (52.5
-// M cells); FP16 39.6 -> 22.7 us (ellipsoid), and on the 10.7 M-cell thermal
-// wing 2 x 65.6 -> 76 us for f and g in one launch.  The two cells of an x row
+// region in LDS (16-bit), one launch of the finest fill: 22.8 -> 16.6 us (FP32
+// sphere, 500 chunks), 44.5 -> 35.5 us (6.1 M-cell cube), 142 -> 122 us (52.5
+// M cells); FP16 39.6 -> 22.9 us (ellipsoid), and on the 10.7 M-cell thermal
+// wing 2 x 65.6 -> 80 us for f and g in one launch.  The two cells of an x row
 // in one store did not change it; 8 waves per SIMD (32 groups of LDS) gave up to
 // 1 % of a step over 7.
 // Parent cell of corner q of a group, as (block << 9 | cell) or -1.  Per axis,
@@ -1364,15 +1364,43 @@ __device__ __forceinline__ int ghost_corner(const LevelArgs& L, int first, uint3
     return pb < 0 ? -1 : (pb << 9) | cell;
 }
 
+// Arithmetic of the fill.  A fused multiply-add chosen by the compiler depends
+// on what surrounds an expression, and one differently rounded ghost value
+// shows in every later step (16-bit storage turns it into a whole unit of the
+// last stored place).  Products that the fast build does not fuse are therefore
+// hidden from it, which leaves one way to contract each sum; the operations
+// and their order are those of feq2 / feq4 / geq and of the reference's blend.
+// Costs 0.3 to 0.8 % of a step against leaving the choice to the compiler.
+__device__ __forceinline__ float own_rounding(float x) {
+    asm("" : "+v"(x));
+    return x;
+}
+
 // Trilinear blend of the 8 corner values with the weights of one fine cell.
+__device__ __forceinline__ float ghost_lerp(float lo, float hi, float w) {
+    return lo * (1.0f - w) + own_rounding(hi * w);
+}
 __device__ __forceinline__ float ghost_blend(const float (&v)[8], float wx, float wy, float wz) {
-    float c00 = v[0] * (1.0f - wx) + v[1] * wx;
-    float c01 = v[4] * (1.0f - wx) + v[5] * wx;
-    float c10 = v[2] * (1.0f - wx) + v[3] * wx;
-    float c11 = v[6] * (1.0f - wx) + v[7] * wx;
-    float c0 = c00 * (1.0f - wy) + c10 * wy;
-    float c1 = c01 * (1.0f - wy) + c11 * wy;
-    return c0 * (1.0f - wz) + c1 * wz;
+    const float c00 = ghost_lerp(v[0], v[1], wx), c01 = ghost_lerp(v[4], v[5], wx);
+    const float c10 = ghost_lerp(v[2], v[3], wx), c11 = ghost_lerp(v[6], v[7], wx);
+    return ghost_lerp(ghost_lerp(c00, c10, wy), ghost_lerp(c01, c11, wy), wz);
+}
+
+// Equilibria of the blended density (temperature) r and velocity.
+__device__ __forceinline__ float ghost_feq(const float4& r, float w, float cx, float cy, float cz, int comp) {
+    const float cu = cz * r.w + (cx * r.y + own_rounding(cy * r.z));
+    const float usq = r.w * r.w + (r.y * r.y + own_rounding(r.z * r.z));
+    const float usq15 = own_rounding(1.5f * usq);
+    if (comp != 1) return own_rounding(r.x * w * (cu * own_rounding(4.5f * cu) + (3.0f * cu + 1.0f) - usq15));
+    const float cu2 = own_rounding(cu * cu), cu3 = own_rounding(cu2 * cu), cu4 = own_rounding(cu2 * cu2);
+    float val = 4.5f * cu2 + (3.0f * cu + 1.0f) - usq15;
+    val += 4.5f * cu3 - own_rounding(4.5f * cu * usq);
+    val += 3.375f * cu4 - own_rounding(6.75f * cu2 * usq) + own_rounding(1.125f * own_rounding(usq * usq));
+    return own_rounding(r.x * w * val);
+}
+__device__ __forceinline__ float ghost_geq(float T, const float4& r, float w, float cx, float cy, float cz) {
+    const float cu = cz * r.w + (cx * r.y + own_rounding(cy * r.z));
+    return own_rounding(w * T * (3.0f * cu + 1.0f));
 }
 
 // Temporal blends (tw = 0 and 0.5) of one field's corner values; a corner the
@@ -1464,16 +1492,17 @@ __device__ __forceinline__ void ghost_store(const GhostArgs& a, const float4 (*m
             out0[dx] = out1[dx] = 0.0f;
             if (bits & (1u << dx)) {
                 const int d = dx + 2 * row;
-                const float wx = ghost_weight(d, 0);
+                float wx = ghost_weight(d, 0);
+                asm("" : "+v"(wx) : "s"(row));  // not hoisted: the blends of all rows would not fit in registers
                 const float rr0 = ghost_blend(f0, wx, wy, wz), rr1 = ghost_blend(f1, wx, wy, wz);
                 const float4 r0 = mac[lg * 8 + d][0], r1 = mac[lg * 8 + d][1];  // density, velocity
                 float eq0, eq1;
                 if constexpr (THERMAL) {
-                    eq0 = geq(mact[lg * 8 + d][0], r0.y, r0.z, r0.w, w_k, cx, cy, cz);
-                    eq1 = geq(mact[lg * 8 + d][1], r1.y, r1.z, r1.w, w_k, cx, cy, cz);
+                    eq0 = ghost_geq(mact[lg * 8 + d][0], r0, w_k, cx, cy, cz);
+                    eq1 = ghost_geq(mact[lg * 8 + d][1], r1, w_k, cx, cy, cz);
                 } else {
-                    eq0 = feq_auto(r0.x, r0.y, r0.z, r0.w, w_k, cx, cy, cz, comp);
-                    eq1 = feq_auto(r1.x, r1.y, r1.z, r1.w, w_k, cx, cy, cz, comp);
+                    eq0 = ghost_feq(r0, w_k, cx, cy, cz, comp);
+                    eq1 = ghost_feq(r1, w_k, cx, cy, cz, comp);
                 }
                 const float neq0 = rr0 - eq0, neq1 = rr1 - eq1;
                 out0[dx] = eq0 + neq0 * scale;
