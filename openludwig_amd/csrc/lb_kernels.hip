@@ -1873,12 +1873,14 @@ __device__ void forces_block(const ForceArgs& a, int64_t chunk) {
     // Triangles whose probes met no fluid: the nearest fluid cell on the
     // normal's side, in the first shell of cells around the triangle that has
     // one (the first such cell in the reference's loop order).  The work-group
-    // lists them and searches each with 16 lanes, one sweep over all shells, a
-    // lane per row of cells with 8 solid flags in one load.  Bound by latency: one work-item per triangle
-    // walking 11^3 cells, each a block lookup and then a flag, held less than
-    // one wave per SIMD for 509 us on the 40,400-triangle wing (400 such
-    // triangles outside, 28,300 inside); now 152 us on average of the two sides,
-    // 15 us as before where no triangle needs it.
+    // lists them and searches each with 16 lanes, a lane per row of cells with 8
+    // solid flags in one load, rows from the inside out until no further row can
+    // hold a nearer shell.  Bound by latency: one work-item per triangle walking
+    // 11^3 cells, each a block lookup and then a flag, held less than one wave
+    // per SIMD for 509 us on the 40,400-triangle wing (400 such triangles
+    // outside, 28,300 inside); 16 lanes over all rows took 152 us on average of
+    // the two sides, stopping at the shell found 132 us.  15 us as before where
+    // no triangle needs it.
     if (tid == 0) n_left = 0;
     __syncthreads();
     if (mine && !found) {
@@ -1896,45 +1898,61 @@ __device__ void forces_block(const ForceArgs& a, int64_t chunk) {
         uint64_t key = ~0ull;  // shell, then squared distance
         int64_t place = INT64_MAX;
         SearchHit hit{-1, 0, 0.0f};
-        const int x0 = max(g_x - R, 1), x1 = min(g_x + R, a.gdx * BS);
-        for (int row = sub; row < side * side; row += 16) {
-            const int dy = row % side - R, dz = row / side - R;
+        int near = INT32_MAX;  // the least shell that any of the 16 lanes has met
+        for (int base = 0, ring = 0; base < side * side; base += 16) {
+            // rows (dy, dz) ring by ring, max(|dy|, |dz|) = ring: a cell of a
+            // row further out than `near` lies in a later shell
+            while ((2 * ring + 1) * (2 * ring + 1) <= base) ring++;
+            if (ring > near) break;
+            const int row = base + sub;
+            int r = ring;
+            while ((2 * r + 1) * (2 * r + 1) <= row) r++;
+            const int o = r > 0 ? row - (2 * r - 1) * (2 * r - 1) : 0, edge = r > 0 ? o / (2 * r) : 0;
+            const int run = o - edge * 2 * r;
+            const int dy = edge == 0 ? run - r : edge == 1 ? r : edge == 2 ? r - run : -r;
+            const int dz = edge == 0 ? -r : edge == 1 ? run - r : edge == 2 ? r : r - run;
             const int cgy = g_y + dy, cgz = g_z + dz;
-            if (cgy < 1 || cgz < 1 || cgy > a.gdy * BS || cgz > a.gdz * BS) continue;
-            const int32_t* grid = a.grid + (size_t)a.gdx * ((size_t)((cgy - 1) >> 3) + (size_t)a.gdy * ((cgz - 1) >> 3));
-            const int line = ((cgy - 1) & 7) * BS + ((cgz - 1) & 7) * BS * BS;
-            const float ccy = ((float)cgy - 0.5f) * a.dx, ccz = ((float)cgz - 0.5f) * a.dx;
-            const float dyp = ccy - q.y, dzp = ccz - q.z;
-            // the row's cells of up to three blocks at a time, 8 flags in one load each
-            for (int bx0 = (x0 - 1) >> 3; bx0 <= (x1 - 1) >> 3; bx0 += 3) {
-                int id[3];
-                uint64_t flags[3];
+            if (r <= R && r <= near && cgy >= 1 && cgz >= 1 && cgy <= a.gdy * BS && cgz <= a.gdz * BS) {
+                const int reach = near < R ? near : R;
+                const int x0 = max(g_x - reach, 1), x1 = min(g_x + reach, a.gdx * BS);
+                const int32_t* grid =
+                    a.grid + (size_t)a.gdx * ((size_t)((cgy - 1) >> 3) + (size_t)a.gdy * ((cgz - 1) >> 3));
+                const int line = ((cgy - 1) & 7) * BS + ((cgz - 1) & 7) * BS * BS;
+                const float ccy = ((float)cgy - 0.5f) * a.dx, ccz = ((float)cgz - 0.5f) * a.dx;
+                const float dyp = ccy - q.y, dzp = ccz - q.z;
+                // the row's cells of up to three blocks at a time, 8 flags in one load each
+                for (int bx0 = (x0 - 1) >> 3; bx0 <= (x1 - 1) >> 3; bx0 += 3) {
+                    int id[3];
+                    uint64_t flags[3];
 #pragma unroll
-                for (int u = 0; u < 3; u++) id[u] = bx0 + u <= (x1 - 1) >> 3 ? grid[bx0 + u] : -1;
+                    for (int u = 0; u < 3; u++) id[u] = bx0 + u <= (x1 - 1) >> 3 ? grid[bx0 + u] : -1;
 #pragma unroll
-                for (int u = 0; u < 3; u++)
-                    flags[u] = id[u] >= 0 ? *(const uint64_t*)(a.obst + (size_t)id[u] * NC + line) : ~0ull;
+                    for (int u = 0; u < 3; u++)
+                        flags[u] = id[u] >= 0 ? *(const uint64_t*)(a.obst + (size_t)id[u] * NC + line) : ~0ull;
 #pragma unroll
-                for (int u = 0; u < 3; u++) {
-                    // bit 8 l + 7 set for each fluid cell l (a zero byte)
-                    const uint64_t low = 0x7f7f7f7f7f7f7f7full;
-                    uint64_t fluid = ~(((flags[u] & low) + low) | flags[u] | low);
-                    for (; fluid != 0; fluid &= fluid - 1) {
-                        const int lx = __builtin_ctzll(fluid) >> 3, cgx = (bx0 + u) * BS + lx + 1;
-                        const int ddx = cgx - g_x;
-                        if (cgx < x0 || cgx > x1) continue;
-                        const int rad = max(abs(ddx), max(abs(dy), abs(dz)));
-                        const float ccx = ((float)cgx - 0.5f) * a.dx;
-                        const float dxp = ccx - q.x;
-                        const float dn = dxp * q.nx + dyp * q.ny + dzp * q.nz;
-                        const float dsq = dxp * dxp + dyp * dyp + dzp * dzp;
-                        const uint64_t k = (uint64_t)(uint32_t)rad << 32 | __float_as_uint(dsq);
-                        // a lane meets its cells in loop order: an equal key does not replace
-                        if (rad > 0 && !(dn <= 0.0f) && dsq < 1e10f && k < key)
-                            key = k, place = (int64_t)row * side + ddx + R, hit = {id[u], line + lx, dn};
+                    for (int u = 0; u < 3; u++) {
+                        // bit 8 l + 7 set for each fluid cell l (a zero byte)
+                        const uint64_t low = 0x7f7f7f7f7f7f7f7full;
+                        uint64_t fluid = ~(((flags[u] & low) + low) | flags[u] | low);
+                        for (; fluid != 0; fluid &= fluid - 1) {
+                            const int lx = __builtin_ctzll(fluid) >> 3, cgx = (bx0 + u) * BS + lx + 1;
+                            const int ddx = cgx - g_x;
+                            if (cgx < x0 || cgx > x1) continue;
+                            const int rad = max(abs(ddx), r);
+                            const float ccx = ((float)cgx - 0.5f) * a.dx;
+                            const float dxp = ccx - q.x;
+                            const float dn = dxp * q.nx + dyp * q.ny + dzp * q.nz;
+                            const float dsq = dxp * dxp + dyp * dyp + dzp * dzp;
+                            const uint64_t k = (uint64_t)(uint32_t)rad << 32 | __float_as_uint(dsq);
+                            const int64_t at = ((int64_t)(dz + R) * side + dy + R) * side + ddx + R;
+                            if (rad > 0 && !(dn <= 0.0f) && dsq < 1e10f && (k < key || (k == key && at < place)))
+                                key = k, place = at, hit = {id[u], line + lx, dn};
+                        }
                     }
                 }
             }
+            near = key == ~0ull ? near : min(near, (int)(key >> 32));
+            for (int off = 8; off > 0; off >>= 1) near = min(near, __shfl_xor(near, off, 16));
         }
         // the least (shell, distance, place) of the 16 lanes
         uint64_t lk = key;
