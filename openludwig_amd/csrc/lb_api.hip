@@ -532,8 +532,8 @@ int profile_begin(lb_ctx* c, Level& L, int which, hipEvent_t* end) {
     return LB_OK;
 }
 
-// Occupancy of the interior stream-collide kernel per population storage:
-// 6 waves per SIMD for 16-bit storage, 5 for FP32.  Measured on the 52.5M-cell
+// Occupancy of the stream-collide kernel per population storage: 6 waves per
+// SIMD for 16-bit storage (small launches take 5, see SMALL_TILES), 5 for FP32.  Measured on the 52.5M-cell
 // cube case through the engine: FP16 11.56 -> 11.17 ms per coarse step at 6;
 // FP32 15.46 ms at either.
 int default_waves(int storage) { return storage == LB_STORAGE_FP32 ? 5 : 6; }

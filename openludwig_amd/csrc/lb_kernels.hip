@@ -1162,6 +1162,16 @@ inline unsigned persistent_groups(int n_tiles) {
     return need < full ? need : full;
 }
 
+// 16-bit launches of up to this many blocks run at 5 waves per SIMD whatever is
+// asked for: two rounds of the chip at 5 work-groups per CU.  There the sixth
+// wave hides nothing, and its spills (71 against 21 registers) lie on the
+// critical path of each work-group.  6 -> 5 waves, per launch: 192 work-groups
+// (two per block) 11.2 -> 10.3 us, 256 11.0 -> 9.6, 1,280 21.8 -> 18.1, 1,536
+// 22.4 -> 20.8, 1,784 28.5 -> 24.2; 3,456 34.0 -> 34.5, 10,816 96.4 -> 97.1,
+// 25,472 214.5 -> 216.9.  FP32 is faster at 5 on every size (27.5 against 30.3
+// at 1,536, 168 against 175 at 14,336) and takes 6 only when asked to.
+constexpr int32_t SMALL_TILES = 1280;
+
 template <int ST, class OffT>
 void collide_launch(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_tiles, int64_t j,
                     int sched, int waves, hipStream_t s) {
@@ -1172,14 +1182,15 @@ void collide_launch(const LevelArgs* las, const CaseState* states, const Work* w
         return;
     }
     const dim3 g(padded_groups(n_tiles));
-    if (waves == 6)
+    if (waves == 6 && !(ST != 0 && n_tiles <= SMALL_TILES))
         hipLaunchKernelGGL((collide_kernel<ST, OffT, 6>), g, t, 0, s, las, states, work, n_tiles, j, sched);
     else
         hipLaunchKernelGGL((collide_kernel<ST, OffT, 5>), g, t, 0, s, las, states, work, n_tiles, j, sched);
 }
 
 // Work entries whose block has a missing neighbour (ghost blocks count as
-// present) carry WORK_BOUNDARY.  waves: occupancy (5 or 6 waves per SIMD).
+// present) carry WORK_BOUNDARY.  waves: occupancy (5 or 6 waves per SIMD; small
+// 16-bit launches take 5).
 hipError_t collide(const LevelArgs* las, const CaseState* states, const Work* work, int32_t n_tiles, int64_t j,
                    int storage, int wide, int sched, int waves, hipStream_t s) {
     if (n_tiles <= 0) return hipSuccess;
