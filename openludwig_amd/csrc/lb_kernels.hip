@@ -1347,12 +1347,13 @@ hipError_t thermal(const LevelArgs* las, const CaseState* states, const Work* wo
 // density and velocity blends of the chunk's groups into LDS, a work-item per
 // (group, field), then a work-item per (group, direction).  Against a
 // work-item per ghost cell (FP32) and per-block staging of the 5^3 parent
-// region in LDS (16-bit), one launch of the finest fill: 22.8 -> 16.6 us (FP32
-// sphere, 500 chunks), 44.5 -> 35.5 us (6.1 M-cell cube), 142 -> 122 us (52.5
-// M cells); FP16 39.6 -> 22.9 us (ellipsoid), and on the 10.7 M-cell thermal
-// wing 2 x 65.6 -> 80 us for f and g in one launch.  The two cells of an x row
-// in one store did not change it; 8 waves per SIMD (32 groups of LDS) gave up to
-// 1 % of a step over 7.
+// region in LDS (16-bit), one launch of the finest fill: 22.8 -> 16.0 us (FP32
+// sphere, 500 chunks), 44.5 -> 34.3 us (6.1 M-cell cube), 142 -> 118 us (52.5
+// M cells); FP16 39.6 -> 21.9 us (ellipsoid), and on the 10.7 M-cell thermal
+// wing 2 x 65.6 -> 72 us for f and g in one launch.  The two cells of an x row
+// in one store did not change it; 32 groups of LDS (7 waves per SIMD) gave up to
+// 1 % of a step over 64.  8 waves spill 2 to 6 registers: 0.2 to 0.7 % of a step
+// slower than 7 (FP16 wing 4.57 -> 4.54 ms), 6 equals 7.
 // Parent cell of corner q of a group, as (block << 9 | cell) or -1.  Per axis,
 // the fine cell centres lie at (x - 0.5) / 2 in parent cells, x = origin +
 // local + 1, so the lower corner is max(1, origin / 2 + m) and the upper one
@@ -1381,7 +1382,8 @@ __device__ __forceinline__ int ghost_corner(const LevelArgs& L, int first, uint3
 // last stored place).  Products that the fast build does not fuse are therefore
 // hidden from it, which leaves one way to contract each sum; the operations
 // and their order are those of feq2 / feq4 / geq and of the reference's blend.
-// Costs 0.3 to 0.8 % of a step against leaving the choice to the compiler.
+// At 7 waves per SIMD this costs nothing against leaving the choice to the
+// compiler (at 8, where it spills, 0.3 to 0.8 % of a step).
 __device__ __forceinline__ float own_rounding(float x) {
     asm("" : "+v"(x));
     return x;
@@ -1534,7 +1536,7 @@ __device__ __forceinline__ void ghost_store(const GhostArgs& a, const float4 (*m
 }
 
 template <int ST>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) ghost_kernel(const LevelArgs* __restrict__ las,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) ghost_kernel(const LevelArgs* __restrict__ las,
                                                     const CaseState* __restrict__ states,
                                                     const Work* __restrict__ work, int64_t j) {
     __shared__ float4 mac[GHOST_GROUPS * 8][2];  // [cell of group][tw = 0, 0.5]: density, velocity
