@@ -416,10 +416,24 @@ int build_links(lb_ctx* c, Level& L, const lb_level_desc* d) {
             cb.push_back(bb);
         }
     }
-    L.nlinks = (int64_t)dst.size();
-    if (L.nlinks == 0) return LB_OK;
-    const size_t n = (size_t)L.nlinks;
-    if (n > (size_t)INT32_MAX) return fail(c, LB_EINVAL, "level %d: %zu wall links", d->level_id, n);
+    L.nlinks = 0;
+    if (dst.empty()) return LB_OK;
+    if (dst.size() > (size_t)INT32_MAX) return fail(c, LB_EINVAL, "level %d: %zu wall links", d->level_id, dst.size());
+    // One link per corrected slot.  A cell listed more than once gives the same
+    // slots again; the last listing counts, as in a loop over the list that
+    // reads the uncorrected populations.  (Two links of one slot could stand
+    // in different work entries, and for q >= 0.5 the slot is its own second
+    // source: whichever entry came later would correct the corrected value.)
+    std::vector<int32_t> by_dst(dst.size());
+    for (size_t i = 0; i < dst.size(); i++) by_dst[i] = (int32_t)i;
+    std::sort(by_dst.begin(), by_dst.end(), [&](int32_t u, int32_t v) {
+        return dst[(size_t)u] != dst[(size_t)v] ? dst[(size_t)u] < dst[(size_t)v] : u > v;
+    });
+    by_dst.erase(std::unique(by_dst.begin(), by_dst.end(),
+                             [&](int32_t u, int32_t v) { return dst[(size_t)u] == dst[(size_t)v]; }),
+                 by_dst.end());
+    const size_t n = by_dst.size();
+    L.nlinks = (int64_t)n;
     // Link order.  Sorted by destination, a wave's links share (block,
     // direction) rows, so its loads and stores of the same row coalesce.  A
     // work entry gathers its links' values before it stores any, so a link that
@@ -427,9 +441,7 @@ int build_links(lb_ctx* c, Level& L, const lb_level_desc* d) {
     // sides, or two cells apart from one) has to be in the same entry: linked
     // links stand together, and entries of up to 256 links are cut between
     // such groups (one longer group makes one longer entry).
-    std::vector<int32_t> by_dst(n), group(n);
-    for (size_t i = 0; i < n; i++) by_dst[i] = (int32_t)i;
-    std::sort(by_dst.begin(), by_dst.end(), [&](int32_t u, int32_t v) { return dst[(size_t)u] < dst[(size_t)v]; });
+    std::vector<int32_t> group(n);
     for (size_t r = 0; r < n; r++) group[r] = (int32_t)r;  // over ranks in by_dst; the root is the lowest rank
     auto root = [&](int32_t r) {
         while (group[(size_t)r] != r) r = group[(size_t)r] = group[(size_t)group[(size_t)r]];
@@ -439,8 +451,8 @@ int build_links(lb_ctx* c, Level& L, const lb_level_desc* d) {
     std::vector<int32_t> block_row((size_t)nb, -1);
     std::vector<uint64_t> bits;
     constexpr size_t kRow = (size_t)Q * NC / 64;
-    for (size_t i = 0; i < n; i++) {
-        const size_t blk = (size_t)dst[i] / (Q * NC), at = (size_t)dst[i] % (Q * NC);
+    for (const int32_t i : by_dst) {
+        const size_t blk = (size_t)dst[(size_t)i] / (Q * NC), at = (size_t)dst[(size_t)i] % (Q * NC);
         if (block_row[blk] < 0) {
             block_row[blk] = (int32_t)(bits.size() / kRow);
             bits.resize(bits.size() + kRow, 0);
