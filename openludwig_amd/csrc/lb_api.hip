@@ -667,12 +667,16 @@ int upload_level_args(lb_ctx* c, int li) {
     A.tau_g = L.tau_g;
     if (li > 0) {
         const Level& P = c->levels[(size_t)li - 1];
+        // The ghost fill reads block 0 of the parent in place of a corner that
+        // the parent level does not hold, and drops what it read.  A parent
+        // without blocks has no block 0 to read; the level's own stands in.
+        const Level& S = P.nb > 0 ? P : L;
         for (int i = 0; i < 2; i++) {
-            A.pf[i] = P.f[i];
-            A.prho[i] = P.rho[i];
-            A.pvel[i] = P.vel[i];
-            A.pg[i] = P.g[i];
-            A.pT[i] = P.T[i];
+            A.pf[i] = S.f[i];
+            A.prho[i] = S.rho[i];
+            A.pvel[i] = S.vel[i];
+            A.pg[i] = S.g[i];
+            A.pT[i] = S.T[i];
         }
         A.ptau = P.tau;
         A.ptau_g = P.tau_g;

@@ -1437,7 +1437,8 @@ __device__ __forceinline__ void ghost_in_time(const int (&at)[8], const float (&
 __device__ __forceinline__ float ghost_weight(int d, int ax) { return ((d >> ax) & 1) ? 0.75f : 0.25f; }
 
 // Component k at the 8 corners, new and old (without temporal interpolation
-// the view's old half is the new one); a missing corner reads slot 0, unused.
+// the view's old half is the new one); a missing corner reads block 0, unused
+// (of the level itself where the parent has no block).
 template <int ST>
 __device__ __forceinline__ void ghost_load(const GhostArgs& a, const int (&at)[8], int k, float (&vn)[8],
                                            float (&vo)[8]) {
