@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -126,7 +127,48 @@ struct Level {
 
 }  // namespace
 
+namespace {
+// Whether a context's or engine's stream may hold steps that nobody has waited
+// for: set before they are queued, cleared when the stream is found idle.
+struct Queued {
+    hipStream_t stream = nullptr;
+    bool steps = false;  // under g_queued.mu
+};
+struct QueuedList {
+    std::mutex mu;
+    std::vector<Queued*> all;
+};
+QueuedList g_queued;
+
+void queued_open(Queued* q, hipStream_t stream) {
+    q->stream = stream;
+    std::lock_guard<std::mutex> lk(g_queued.mu);
+    g_queued.all.push_back(q);
+}
+void queued_close(Queued* q) {  // before the stream is destroyed
+    std::lock_guard<std::mutex> lk(g_queued.mu);
+    g_queued.all.erase(std::remove(g_queued.all.begin(), g_queued.all.end(), q), g_queued.all.end());
+}
+void queued_steps(Queued* q) {
+    std::lock_guard<std::mutex> lk(g_queued.mu);
+    q->steps = true;
+}
+bool others_queued(const Queued* self) {
+    std::lock_guard<std::mutex> lk(g_queued.mu);
+    for (Queued* q : g_queued.all) {
+        if (q == self || !q->steps) continue;
+        if (hipStreamQuery(q->stream) != hipSuccess) {
+            (void)hipGetLastError();  // "not ready" is no error of the launches that follow
+            return true;
+        }
+        q->steps = false;
+    }
+    return false;
+}
+}  // namespace
+
 struct lb_ctx {
+    Queued queued;
     int device = 0;
     lb_config cfg{};
     hipStream_t stream = nullptr;
@@ -152,7 +194,7 @@ struct lb_ctx {
     std::vector<lbk::LevelArgs> las_host;
     lb_engine* engine = nullptr;  // set while attached to a batched engine
     bool dry = false;             // footprint planning: nothing is allocated or copied
-    bool counted = false;         // holds a share of the download ring
+    bool counted = false;         // holds a share of the download pieces
 };
 
 // One attached case of an engine.
@@ -184,6 +226,7 @@ struct DepthWork {
 };
 
 struct lb_engine {
+    Queued queued;
     int device = 0;
     int32_t storage = 0;
     const Kern* k = &kStrict;
@@ -976,108 +1019,186 @@ __global__ void stats_reduce_kernel(const double* __restrict__ part, int rows, d
 // into pageable memory and the permutation there by one thread ran at 3 to 5
 // GB/s -- page faults of both arrays, then the copy -- against 18 GB/s now for
 // 1.3 M cells and 44 GB/s for 52.5 M: velocity 4.4 -> 0.9 ms and 204 -> 14 ms.)
-// The pinned pieces are one
-// ring of up to 32 MiB for the process, held while a download runs, grown on
-// demand and freed with the last context.
+// While another context or an engine has steps queued, the pieces come over as
+// copies of the blocks as they lie, and the threads reorder and decode them: a
+// process has 4 hardware queues for all of its streams, so the kernel of an
+// idle context may stand behind everything that a busy one has queued (260 ms
+// behind 3,000 coarse steps of 1.3 M cells, for 2 of 16 contexts; as a copy
+// 0.1 ms), and an event behind a copy would too.  Otherwise the kernel: copies
+// need a quarter to a half longer for 1.3 to 52.5 M cells, and up to 0.1 ms
+// more for each of the smallest (55 k cells).
+// The pinned memory is 8 pieces of 4 MiB for the process, allocated when first
+// needed and given back with the last context.  A piece is held while it is
+// filled and read, never while a context's earlier work is waited for, so
+// downloads of different contexts run side by side; the pieces go round in the
+// order of asking.  No piece is freed while a context lives: hipHostFree waits
+// for everything queued on the device (340 ms behind 1,500 such steps, where
+// hipHostMalloc takes 0.2 ms).
 namespace {
 constexpr size_t kPiece = (size_t)4 << 20;  // bytes; a multiple of a 512-float row
 constexpr int kPieces = 8;
 
-struct Staging {
-    std::mutex mu;  // one download at a time
+struct Piece {
     float* buf = nullptr;
-    int pieces = 0;
-    size_t piece = 0;  // bytes of each
+    size_t bytes = 0;
+    bool held = false;
+};
+struct Staging {
+    std::mutex mu;  // held for these fields alone, not over a call to the device
+    std::condition_variable cv;
+    Piece piece[kPieces];
+    uint64_t asked = 0, served = 0;
     int contexts = 0;
 };
 Staging g_staging;
 
-void staging_free_locked() {
-    if (g_staging.buf) (void)hipHostFree(g_staging.buf);
-    g_staging.buf = nullptr;
-    g_staging.pieces = 0;
-    g_staging.piece = 0;
-}
-
 void staging_context(int change) {
-    std::lock_guard<std::mutex> lk(g_staging.mu);
-    g_staging.contexts += change;
-    if (g_staging.contexts <= 0) staging_free_locked();
+    float* spare[kPieces];
+    int n = 0;
+    {
+        std::lock_guard<std::mutex> lk(g_staging.mu);
+        g_staging.contexts += change;
+        if (g_staging.contexts > 0) return;
+        for (Piece& p : g_staging.piece) {
+            if (p.held || !p.buf) continue;
+            spare[n++] = p.buf;
+            p.buf = nullptr;
+            p.bytes = 0;
+        }
+    }
+    for (int i = 0; i < n; i++) (void)hipHostFree(spare[i]);
 }
 
-// A ring for `bytes` of output; less than asked for when memory is short.
-int staging_reserve_locked(lb_ctx* c, size_t bytes) {
-    size_t piece = kPiece;
-    int pieces = kPieces;
-    if (bytes < kPiece) {  // one piece, a power of two of rows
-        pieces = 1;
-        while (piece / 2 >= bytes && piece > 65536) piece /= 2;
-    } else {
-        while (pieces > 1 && kPiece * (size_t)(pieces / 2) >= bytes) pieces /= 2;
-    }
-    if (g_staging.piece * (size_t)g_staging.pieces >= piece * (size_t)pieces) return LB_OK;
-    staging_free_locked();
-    for (;;) {
-        const hipError_t e = hipHostMalloc((void**)&g_staging.buf, piece * (size_t)pieces, hipHostMallocPortable);
-        if (e == hipSuccess) break;
-        g_staging.buf = nullptr;
-        (void)hipGetLastError();
-        if (pieces > 1) pieces /= 2;
-        else if (piece > 65536) piece /= 2;
-        else return fail(c, LB_ENOMEM, "hipHostMalloc(%zu bytes) failed: %s", piece, hipGetErrorString(e));
-    }
-    g_staging.piece = piece;
-    g_staging.pieces = pieces;
-    return LB_OK;
+// The next free piece, one that has its memory if there is any.
+Piece* staging_take() {
+    std::unique_lock<std::mutex> lk(g_staging.mu);
+    const uint64_t turn = g_staging.asked++;
+    Piece* p = nullptr;
+    g_staging.cv.wait(lk, [&] {
+        if (turn != g_staging.served) return false;
+        for (Piece& q : g_staging.piece)
+            if (!q.held && (!p || (!p->buf && q.buf))) p = &q;
+        return p != nullptr;
+    });
+    p->held = true;
+    g_staging.served++;
+    lk.unlock();
+    g_staging.cv.notify_all();
+    return p;
 }
 
-int download_field(lb_ctx* c, const Level& L, const void* src, int n_comp, int storage, float* dst) {
-    const int64_t rows = (int64_t)L.nb * n_comp;
-    if (rows == 0) return LB_OK;
-    std::lock_guard<std::mutex> lk(g_staging.mu);
-    RC(staging_reserve_locked(c, (size_t)rows * NC * 4));
-    const int64_t per = (int64_t)(g_staging.piece / (NC * 4));  // rows of a piece
-    const int64_t n_pieces = (rows + per - 1) / per;
-    const int workers = (int)std::min<int64_t>(g_staging.pieces, n_pieces);
+void staging_give(Piece* p) {
+    {
+        std::lock_guard<std::mutex> lk(g_staging.mu);
+        p->held = false;
+    }
+    g_staging.cv.notify_all();
+}
+
+// Memory for a piece in hand; less than a whole piece when memory is short.
+hipError_t staging_fill(Piece* p) {
+    hipError_t e = hipSuccess;
+    for (size_t bytes = kPiece; !p->buf && bytes >= 65536; bytes /= 2) {
+        e = hipHostMalloc((void**)&p->buf, bytes, hipHostMallocPortable);
+        if (e == hipSuccess) {
+            p->bytes = bytes;
+        } else {
+            p->buf = nullptr;
+            (void)hipGetLastError();
+        }
+    }
+    return p->buf ? hipSuccess : e;
+}
+
+// A row of 512 populations as the device stores it, decoded (lb_kernels.hip,
+// Codec): w_k + the stored value.  FP16 without FP32 subnormals on the way, so
+// that a thread's flush mode does not matter.
+void decode_row(const uint8_t* src, int storage, float w, float* out) {
+    if (storage == LB_STORAGE_FP32) {
+        std::memcpy(out, src, (size_t)NC * 4);
+        return;
+    }
+    uint16_t h[NC];
+    std::memcpy(h, src, sizeof h);
+    for (int i = 0; i < NC; i++) {
+        uint32_t bits;
+        if (storage == LB_STORAGE_BF16) {
+            bits = (uint32_t)h[i] << 16;
+        } else {
+            const uint32_t a = (uint32_t)(h[i] & 0x7fffu) << 13, e = a & 0x0f800000u;
+            // exponent 0: 2^-14 (1 + m) - 2^-14; 31: inf and NaN
+            const float small = __builtin_bit_cast(float, a + 0x38800000u) - 6.103515625e-05f;
+            const uint32_t b = e == 0u ? __builtin_bit_cast(uint32_t, small)
+                                       : a + (e == 0x0f800000u ? 0x70000000u : 0x38000000u);
+            bits = b | (uint32_t)(h[i] & 0x8000u) << 16;
+        }
+        out[i] = w + __builtin_bit_cast(float, bits);
+    }
+}
+
+// Field `src` of n_comp components to dst (component k of the caller's block i
+// at row k nb + i).  The context's stream is idle on entry.
+int download_field(lb_ctx* c, const Level& L, const void* src, int n_comp, int storage, bool population, float* dst) {
+    const int64_t nb = L.nb;
+    if (nb == 0) return LB_OK;
+    const bool copies = others_queued(&c->queued);
+    const size_t row = (size_t)NC * pop_bytes(storage);
+    // what a piece is filled with: device blocks, or rows of the caller's array
+    const size_t unit = copies ? row * (size_t)n_comp : (size_t)NC * 4;
+    const int64_t units = copies ? nb : nb * n_comp;
+    const int workers = (int)std::min<uint64_t>(kPieces, ((uint64_t)units * unit + kPiece - 1) / kPiece);
     std::mutex launch;
+    std::atomic<int64_t> next{0};  // first unit that no worker has
     std::atomic<int> err{(int)hipSuccess};
-    // Worker w takes pieces w, w + workers, ... through its own part of the
-    // ring: launch, wait for that launch, copy.  The launches share the case's
-    // stream, so a piece is written while the workers before it copy.
-    auto work = [&](int w) noexcept {
-        float* const buf = g_staging.buf + (size_t)w * (g_staging.piece / 4);
+    // A worker takes a piece, has the next units put into it, and stores them.
+    // All use the case's stream, so a piece is filled while the other workers
+    // empty theirs.
+    auto work = [&]() noexcept {
         hipEvent_t done = nullptr;
         hipError_t e = hipSetDevice(c->device);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&done, hipEventDisableTiming);
-        for (int64_t p = w; e == hipSuccess && p < n_pieces && err.load() == (int)hipSuccess; p += workers) {
-            const int64_t r0 = p * per, n = std::min(per, rows - r0);
-            {
-                std::lock_guard<std::mutex> ll(launch);
-                e = c->k->export_rows(src, L.inv, L.nb, n_comp, storage, r0, (int32_t)n, buf, c->stream);
-                if (e == hipSuccess) e = hipEventRecord(done, c->stream);
+        // (one worker: its launches are all that the stream holds)
+        if (e == hipSuccess && workers > 1 && !copies) e = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+        while (e == hipSuccess && err.load() == (int)hipSuccess && next.load() < units) {
+            Piece* const p = staging_take();
+            e = staging_fill(p);
+            const int64_t per = (int64_t)(p->bytes / unit), u0 = e == hipSuccess ? next.fetch_add(per) : units,
+                          n = std::min(per, units - u0);
+            if (n > 0 && copies) {
+                e = hipMemcpyWithStream(p->buf, (const uint8_t*)src + (size_t)u0 * unit, (size_t)n * unit,
+                                        hipMemcpyDeviceToHost, c->stream);
+                for (int64_t b = 0; e == hipSuccess && b < n; b++)
+                    for (int k = 0; k < n_comp; k++)
+                        decode_row((const uint8_t*)p->buf + (size_t)b * unit + (size_t)k * row, storage,
+                                   population ? wk_host(k) : 0.0f,
+                                   dst + ((size_t)k * (size_t)nb + (size_t)L.perm[(size_t)(u0 + b)]) * NC);
+            } else if (n > 0) {
+                {
+                    std::lock_guard<std::mutex> ll(launch);
+                    e = c->k->export_rows(src, L.inv, L.nb, n_comp, storage, u0, (int32_t)n, p->buf, c->stream);
+                    if (e == hipSuccess && done) e = hipEventRecord(done, c->stream);
+                }
+                if (e == hipSuccess) e = done ? hipEventSynchronize(done) : hipStreamSynchronize(c->stream);
+                if (e == hipSuccess) std::memcpy(dst + (size_t)u0 * NC, p->buf, (size_t)n * unit);
             }
-            if (e == hipSuccess) e = hipEventSynchronize(done);
-            if (e == hipSuccess) std::memcpy(dst + (size_t)r0 * NC, buf, (size_t)n * NC * 4);
+            if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);  // nothing writes a piece once it is given back
+            staging_give(p);
         }
         if (done) (void)hipEventDestroy(done);
         if (e != hipSuccess) err.store((int)e);
     };
-    std::vector<std::thread> threads;
-    std::vector<int> here{0};  // workers that run on this thread
-    for (int w = 1; w < workers; w++) {
+    std::thread threads[kPieces - 1];
+    for (int w = 0; w + 1 < workers; w++) {
         try {
-            threads.emplace_back(work, w);
-        } catch (...) {  // no thread to be had
-            here.push_back(w);
+            threads[w] = std::thread(work);
+        } catch (...) {  // no thread to be had: the others take its share
         }
     }
-    for (int w : here) work(w);
-    for (std::thread& t : threads) t.join();
+    work();
+    for (std::thread& t : threads)
+        if (t.joinable()) t.join();
     const hipError_t e = (hipError_t)err.load();
-    if (e != hipSuccess) {
-        (void)hipStreamSynchronize(c->stream);  // nothing writes the ring once it is released
-        return fail(c, LB_EHIP, "field download: %s", hipGetErrorString(e));
-    }
+    if (e != hipSuccess)
+        return fail(c, e == hipErrorOutOfMemory ? LB_ENOMEM : LB_EHIP, "field download: %s", hipGetErrorString(e));
     return LB_OK;
 }
 }  // namespace
@@ -1126,6 +1247,7 @@ int lb_create(lb_ctx** out, int device, const lb_config* cfg) {
         lb_destroy(c);
         return LB_ENOMEM;
     }
+    queued_open(&c->queued, c->stream);
     staging_context(1);
     c->counted = true;
     *out = c;
@@ -1144,6 +1266,7 @@ void lb_destroy(lb_ctx* c) {
                 (void)hipEventDestroy(e.second);
             }
     if (c->stream) {
+        queued_close(&c->queued);
         for (void* p : c->allocs) (void)hipFreeAsync(p, c->stream);
         (void)hipStreamSynchronize(c->stream);
         (void)hipStreamDestroy(c->stream);
@@ -1508,6 +1631,7 @@ int lb_step_batch(lb_ctx* c, int64_t t_start, int32_t n_steps, float u_curr, con
     // One record for the whole call: coarse step t_start + i starts at substep
     // i of level 1.  A record per coarse step was a launch of 5 us each (of 42
     // us for 55 k cells, 330 us for 1.3 M).
+    if (n_steps > 0) queued_steps(&c->queued);
     if (n_steps > 0) HIPCHK(c, c->k->set_state(c->st_dev, case_record(t_start, u_curr, p, c->cfg), c->stream));
     for (int32_t i = 0; i < n_steps; i++) {
         RC(step_level(c, 0, i));
@@ -1659,14 +1783,17 @@ int lb_download_level(lb_ctx* c, int level_id, int field, float* dst) {
     if (!dst || level_id < 1 || level_id > (int)c->levels.size()) return fail(c, LB_EINVAL, "bad arguments");
     HIPCHK(c, hipSetDevice(c->device));
     const Level& L = c->levels[(size_t)level_id - 1];
+    HIPCHK(c, hipStreamSynchronize(c->stream));
     const void* src = nullptr;
     int n_comp = 1, storage = LB_STORAGE_FP32;
+    bool population = false;
     switch (field) {
         case LB_FIELD_F:
         case LB_FIELD_G:
             src = field == LB_FIELD_F ? L.f[L.cur] : L.g[L.cur];
             n_comp = Q;
             storage = c->cfg.storage;
+            population = true;
             break;
         case LB_FIELD_RHO:
             src = L.rho[L.cur];
@@ -1682,7 +1809,7 @@ int lb_download_level(lb_ctx* c, int level_id, int field, float* dst) {
             return fail(c, LB_EINVAL, "unknown field %d", field);
     }
     if (!src) return fail(c, LB_EINVAL, "field not allocated");
-    return download_field(c, L, src, n_comp, storage, dst);
+    return download_field(c, L, src, n_comp, storage, population, dst);
 }
 
 // Overwrite the current state of a level (both halves of the ping-pong pair,
@@ -1867,6 +1994,7 @@ int lb_engine_create(lb_engine** out, int device, int32_t storage, int32_t stric
         delete e;
         return LB_EHIP;
     }
+    queued_open(&e->queued, e->stream);
     *out = e;
     return LB_OK;
 }
@@ -1880,6 +2008,7 @@ void lb_engine_destroy(lb_engine* e) {
     engine_free_lists(e);
     if (e->fin_ents) (void)hipFree(e->fin_ents);
     if (e->fin_counts) (void)hipFree(e->fin_counts);
+    queued_close(&e->queued);
     (void)hipStreamDestroy(e->stream);
     delete e;
 }
@@ -1939,6 +2068,7 @@ int lb_engine_step(lb_engine* e, int32_t n) {
         lbsync::SetupGuard guard;
         RC(engine_rebuild(e));
     }
+    queued_steps(&e->queued);
     if (e->use_graph && !e->exec) {
         // GPU calls of other threads wait for the capture (lb_sync.h);
         // relaxed mode in addition lets them run host-side work meanwhile
