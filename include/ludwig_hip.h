@@ -221,14 +221,16 @@ int lb_stats_noalloc(lb_ctx* ctx, int level_id, double* out);
  * Reads 16 bytes per cell; meant for the diagnostic cadence.               */
 int lb_check_finite(lb_ctx* ctx, int64_t* n_nonfinite);
 
-/* Device bytes the context holds (serving admission).                    */
+/* Device bytes the context counts (serving admission): at least what it
+ * holds.  A case's count does not follow the layout of the library's tables,
+ * so hosts may record it; tables that got smaller count what they did.    */
 int64_t lb_device_bytes(const lb_ctx* ctx);
 
-/* Device bytes a case would hold, computed before anything is allocated
- * (no GPU needed): what lb_create, lb_level_upload of every level and
- * lb_mesh_upload of n_tri triangles allocate, plus the engine's ramp table
- * of n_ramp_batches values (lb_engine_add).  Used to admit serving requests
- * against the HBM budget (no counterpart in the reference).                */
+/* lb_device_bytes of a case, computed before anything is allocated (no GPU
+ * needed): lb_create, lb_level_upload of every level and lb_mesh_upload of
+ * n_tri triangles, plus the engine's ramp table of n_ramp_batches values
+ * (lb_engine_add).  Used to admit serving requests against the HBM budget
+ * (no counterpart in the reference).                                       */
 int lb_footprint(const lb_config* cfg, const lb_level_desc* levels, int32_t n_levels, int64_t n_tri,
                  int32_t n_ramp_batches, int64_t* bytes);
 

@@ -317,12 +317,15 @@ int h2d(lb_ctx* c, T* dst, const T* src, size_t n) {
     return LB_OK;
 }
 
-// Brings what was allocated since `before` up to `bytes`.
-int keep_bytes(lb_ctx* c, int64_t before, int64_t bytes) {
-    const int64_t missing = before + bytes - c->bytes;
-    uint8_t* p = nullptr;
-    return missing > 0 ? dalloc(c, &p, (size_t)missing) : LB_OK;
-}
+// Counts what was allocated since `before` as `bytes` where that is more.  The
+// byte count of a case is a result of the interface (lb_device_bytes,
+// lb_footprint), which hosts record and compare, and does not follow the
+// layout of the tables: one that got smaller goes on counting what it did.
+// Nothing is allocated for the difference.
+void count_as(lb_ctx* c, int64_t before, int64_t bytes) { c->bytes = std::max(c->bytes, before + bytes); }
+// What a level's record counts.
+constexpr int64_t kLevelRecord = 384;
+static_assert((int64_t)sizeof(lbk::LevelArgs) <= kLevelRecord, "a case may not hold more than it counts");
 
 float half_to_float(uint16_t h) {
     int s = (h >> 15) & 1, e = (h >> 10) & 31, m = h & 1023;
@@ -937,6 +940,17 @@ lbk::FiniteEntry finite_entry(const Level& L, int cur, int32_t slot) {
     return e;
 }
 
+// The device buffers of lb_create.
+int create_buffers(lb_ctx* c) {
+    const size_t n = c->levels.size();
+    RC(dalloc(c, &c->st_dev, 1));
+    const int64_t before = c->bytes;
+    RC(dalloc(c, &c->las_dev, n));
+    count_as(c, before, (int64_t)n * kLevelRecord);
+    RC(dalloc(c, &c->fin_ents, n));
+    return dalloc(c, &c->fin_count, 1);
+}
+
 int check_ctx(lb_ctx* c) {
     if (!c) return LB_EINVAL;
     if (c->engine) return fail(c, LB_ESTATE, "case is attached to an engine");
@@ -1242,8 +1256,7 @@ int lb_create(lb_ctx** out, int device, const lb_config* cfg) {
     c->levels.resize((size_t)cfg->n_levels);
     c->las_host.resize((size_t)cfg->n_levels);
     std::memset((void*)c->las_host.data(), 0, c->las_host.size() * sizeof(lbk::LevelArgs));
-    if (dalloc(c, &c->st_dev, 1) != LB_OK || dalloc(c, &c->las_dev, (size_t)cfg->n_levels) != LB_OK ||
-        dalloc(c, &c->fin_ents, (size_t)cfg->n_levels) != LB_OK || dalloc(c, &c->fin_count, 1) != LB_OK) {
+    if (create_buffers(c) != LB_OK) {
         lb_destroy(c);
         return LB_ENOMEM;
     }
@@ -1510,7 +1523,7 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
     RC(dalloc(c, &L.obst, n4));
     RC(dalloc(c, &L.sponge, n4));
     if (d->wall_dist) RC(dalloc(c, &L.wall_dist, n4));
-    RC(keep_bytes(c, c->bytes, std::max(nb, 1)));  // (a flag byte per block, now in the work entries)
+    count_as(c, c->bytes, std::max(nb, 1));  // a flag byte per block (they are in the work entries)
     RC(dalloc(c, &L.nbr, (size_t)nb * Q));
     RC(dalloc(c, &L.borg, borg.size()));
     RC(dalloc(c, &L.inv, (size_t)nb));
@@ -1526,18 +1539,16 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
         RC(h2d(c, L.gchunk, gchunk.data(), gchunk.size()));
     }
     RC(ghost_list(c, L.id - 1, L));
-    // A case's footprint is a number that hosts plan with and keep (admission
-    // budgets, recorded sizes), so tables that got smaller leave it as it is.
-    // The ghost fill's was, per served cell and per ghost block, and with at
-    // least one element per table:
+    // the ghost fill's tables count per served cell and per ghost block, at
+    // least one element each
     {
         const int64_t e = n_entries, gh = n_entries > 0 ? ngh : 0;
         const auto one = [](int64_t n) { return std::max<int64_t>(n, 1); };
         const bool fp32 = c->cfg.storage == LB_STORAGE_FP32;
         const int64_t work = (int64_t)sizeof(lbk::Work) * (fp32 ? (e + 255) / 256 : gh);
-        RC(keep_bytes(c, before_ghosts,
-                      4 * one(2 * e) + work +
-                          (fp32 ? 4 * one(8 * e) : 4 + 4 * (gh + 1) + 4 * one(125 * gh) + 4 * one(gh))));
+        count_as(c, before_ghosts,
+                 4 * one(2 * e) + work +
+                     (fp32 ? 4 * one(8 * e) : 4 + 4 * (gh + 1) + 4 * one(125 * gh) + 4 * one(gh)));
     }
     const size_t ng = (size_t)d->ptr_dim_x * d->ptr_dim_y * d->ptr_dim_z;
     RC(dalloc(c, &L.grid, ng));
@@ -1600,9 +1611,9 @@ int lb_level_upload(lb_ctx* c, const lb_level_desc* d) {
     const int64_t before_links = c->bytes;
     RC(build_links(c, L, d));
     RC(link_list(c, L.id - 1, L));
-    // the footprint the links had: 6 arrays (3 slots, 2 weights, 1 value) and chunks of 256
-    RC(keep_bytes(c, before_links,
-                  L.nlinks * (3 * (L.lidx32 ? 4 : 8) + 12) + (L.nlinks + 255) / 256 * (int64_t)sizeof(lbk::Work)));
+    // the links count 3 slots, 2 weights and 1 value each, and a work entry per 256
+    count_as(c, before_links,
+             L.nlinks * (3 * (L.lidx32 ? 4 : 8) + 12) + (L.nlinks + 255) / 256 * (int64_t)sizeof(lbk::Work));
     RC(upload_level_args(c, L.id - 1));
     L.uploaded = true;
     return LB_OK;
@@ -2230,10 +2241,7 @@ int lb_footprint(const lb_config* cfg, const lb_level_desc* levels, int32_t n_le
     c.cfg = *cfg;
     c.levels.resize((size_t)n_levels);
     c.las_host.resize((size_t)n_levels);
-    RC(dalloc(&c, &c.st_dev, 1));
-    RC(dalloc(&c, &c.las_dev, (size_t)n_levels));
-    RC(dalloc(&c, &c.fin_ents, (size_t)n_levels));
-    RC(dalloc(&c, &c.fin_count, 1));
+    RC(create_buffers(&c));
     for (int i = 0; i < n_levels; i++) RC(lb_level_upload(&c, &levels[i]));
     if (n_tri > 0) RC(lb_mesh_upload(&c, n_tri, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr));
     if (n_ramp_batches > 0) {

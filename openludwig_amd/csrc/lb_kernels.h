@@ -117,7 +117,6 @@ struct LevelArgs {
     const uint32_t* ggroup;
     const uint32_t* gpair;
     BouzidiLinks links;
-    int64_t reserved[11];  // the record's size is part of a case's footprint
 };
 
 // Work list entry.  The neighbour row travels with the entry so that the

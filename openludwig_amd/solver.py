@@ -156,7 +156,7 @@ def lb_config(cfg: CaseConfig, grids: list, params: DomainParameters, storage: i
 
 def footprint(cfg: CaseConfig, grids: list, params: DomainParameters, mesh: SolverMesh | None,
               storage: int = N.LB_STORAGE_FP32, n_ramp_batches: int = 0) -> int:
-    """Exact device bytes of a case (lb_footprint), computed without a GPU."""
+    """Device bytes that a case counts (lb_footprint), computed without a GPU."""
     lib = N.hip_lib()
     keep: list = []
     descs = (N.LbLevelDesc * len(grids))(*[level_desc(g, keep) for g in grids])
