@@ -81,6 +81,18 @@ def log(msg: str) -> None:
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
 
 
+def serving_line(serving: dict | None) -> dict | None:
+    """The serving results as the output line carries them: without the
+    records of the single requests, which go to stderr, one a line.  (With 64
+    of them the line is over 25 kB long and is cut where output is kept by its
+    last few kB.)"""
+    if serving is None:
+        return None
+    for r in serving["per_request"]:
+        log("request " + json.dumps(r))
+    return {k: v for k, v in serving.items() if k != "per_request"}
+
+
 def cpu_baseline(cfg, grids, params, mesh, n_steps: int, diag: int) -> dict:
     """The CPU baseline: the C oracle (FP32 mirror of the restated reference
     algorithm, OpenMP over blocks) on the host cores over coarse steps
@@ -352,7 +364,7 @@ def main() -> int:
                      "traffic_GBps": round(traffic / (avg_ms * 1e-3) / 1e9, 1) if traffic else None,
                      "probe": probe},
         "cpu_baseline": cpu,
-        "serving": serving,
+        "serving": serving_line(serving),
     }
     print(json.dumps(line), flush=True)
     return 0
