@@ -153,8 +153,10 @@ void queued_steps(Queued* q) {
     std::lock_guard<std::mutex> lk(g_queued.mu);
     q->steps = true;
 }
-bool others_queued(const Queued* self) {
+// (self's stream has been waited for)
+bool others_queued(Queued* self) {
     std::lock_guard<std::mutex> lk(g_queued.mu);
+    self->steps = false;
     for (Queued* q : g_queued.all) {
         if (q == self || !q->steps) continue;
         if (hipStreamQuery(q->stream) != hipSuccess) {
@@ -470,14 +472,13 @@ int build_links(lb_ctx* c, Level& L, const lb_level_desc* d) {
     // reads the uncorrected populations.  (Two links of one slot could stand
     // in different work entries, and for q >= 0.5 the slot is its own second
     // source: whichever entry came later would correct the corrected value.)
-    std::vector<int32_t> by_dst(dst.size());
-    for (size_t i = 0; i < dst.size(); i++) by_dst[i] = (int32_t)i;
-    std::sort(by_dst.begin(), by_dst.end(), [&](int32_t u, int32_t v) {
-        return dst[(size_t)u] != dst[(size_t)v] ? dst[(size_t)u] < dst[(size_t)v] : u > v;
-    });
-    by_dst.erase(std::unique(by_dst.begin(), by_dst.end(),
-                             [&](int32_t u, int32_t v) { return dst[(size_t)u] == dst[(size_t)v]; }),
-                 by_dst.end());
+    std::vector<std::pair<int64_t, int32_t>> listed(dst.size());  // slot, minus the place in the list
+    for (size_t i = 0; i < dst.size(); i++) listed[i] = {dst[i], -(int32_t)i};
+    std::sort(listed.begin(), listed.end());
+    std::vector<int32_t> by_dst;
+    by_dst.reserve(listed.size());
+    for (size_t i = 0; i < listed.size(); i++)
+        if (i == 0 || listed[i].first != listed[i - 1].first) by_dst.push_back(-listed[i].second);
     const size_t n = by_dst.size();
     L.nlinks = (int64_t)n;
     // Link order.  Sorted by destination, a wave's links share (block,
