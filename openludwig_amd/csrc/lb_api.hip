@@ -592,9 +592,11 @@ int profile_begin(lb_ctx* c, Level& L, int which, hipEvent_t* end) {
 }
 
 // Occupancy of the stream-collide kernel per population storage: 6 waves per
-// SIMD for 16-bit storage (small launches take 5, see SMALL_TILES), 5 for FP32.  Measured on the 52.5M-cell
-// cube case through the engine: FP16 11.56 -> 11.17 ms per coarse step at 6;
-// FP32 15.46 ms at either.
+// SIMD for 16-bit storage (launches of up to 1,280 blocks take 5 all the same,
+// SMALL_TILES in lb_kernels.hip), 5 for FP32.  Measured through the engine, 5
+// and 6 waves: FP16 1,434 and 1,428 us a coarse step (6.1 M cells), 2,389 and
+// 2,425 (11.4 M, where interior and boundary blocks apart had 2,646 and 2,585),
+// 4,503 and 4,501 (10.7 M, thermal); FP32 1,957 and 2,046 (6.1 M).
 int default_waves(int storage) { return storage == LB_STORAGE_FP32 ? 5 : 6; }
 
 int step_level(lb_ctx* c, int li, int64_t j) {

@@ -689,7 +689,14 @@ __device__ __forceinline__ void vel_tile_store(const VelTile& t, int c, float* v
 // 1.74 -> 1.65 ms (4.5 M cells, thermal); 2.09 -> 2.04 ms at 6.1 M cells.  The
 // two instances are kept apart because one body with the fix-up inside made
 // the 16-bit interior path a third slower (the populations' registers become
-// one tuple that is copied).
+// one tuple that is copied).  They share one register allocation all the same,
+// so a level without boundary blocks runs with the larger one's: FP16 at 6 waves
+// spills 70 VGPRs (39 with the interior instance alone), FP32 at 5 waves 20 (8)
+// and at 6 waves 74 (36), the persistent form 25 and 26 (13).  The finest
+// launches of such levels take what they took before: 212.1 and 213.8 us (FP16,
+// 25,472 work-groups), 231.4 and 232.5 (FP16, 28,416), 124.2 and 124.8 (FP32,
+// 10,240).  FP32 at 6 waves was as fast as at 5 and is now slower: 2,046 against
+// 1,957 us a coarse step (6.1 M cells), 323 against 312 (1.3 M).
 //
 // collide_tile is one half-block tile (work-list entry wk, half `half`);
 // collide_kernel runs one tile per work-group, collide_kernel_persistent
@@ -1062,10 +1069,11 @@ __device__ __forceinline__ void collide_body(const CollideArgs& a, CollideLds<ST
                 alpha = fmaxf(alpha, 0.0f);
                 // The equilibria are computed again rather than kept from
                 // the loop above: kept, they and their terms stay live across
-                // both loops and spill (the interior kernel spilled 63 VGPRs,
-                // 8 without them, and 6 waves per SIMD became the faster
-                // occupancy for 16-bit storage).  Opaque copies of the inputs
-                // stop the compiler from reusing the first loop's values.
+                // both loops and spill (the interior instance alone, FP32 at 5
+                // waves: 63 VGPRs, 8 without them, and 6 waves per SIMD became
+                // the faster occupancy for 16-bit storage).  Opaque copies of
+                // the inputs stop the compiler from reusing the first loop's
+                // values.
                 float r2 = rho, ux2 = uxe, uy2 = uye, uz2 = uze;
                 asm volatile("" : "+v"(r2), "+v"(ux2), "+v"(uy2), "+v"(uz2));
 #pragma unroll
@@ -1164,7 +1172,7 @@ inline unsigned persistent_groups(int n_tiles) {
 
 // 16-bit launches of up to this many blocks run at 5 waves per SIMD whatever is
 // asked for: two rounds of the chip at 5 work-groups per CU.  There the sixth
-// wave hides nothing, and its spills (71 against 21 registers) lie on the
+// wave hides nothing, and its spills (70 against 17 registers) lie on the
 // critical path of each work-group.  6 -> 5 waves, per launch: 192 work-groups
 // (two per block) 11.2 -> 10.3 us, 256 11.0 -> 9.6, 1,280 21.8 -> 18.1, 1,536
 // 22.4 -> 20.8, 1,784 28.5 -> 24.2; 3,456 34.0 -> 34.5, 10,816 96.4 -> 97.1,
@@ -1294,6 +1302,10 @@ __device__ __forceinline__ void thermal_body(const ThermalArgs& a, ThermalLds<ST
     stream_tile<ST, 27>(a.g_out, b, c, G, lds.out + wv * (27 * 64));
 }
 
+// Occupancy: FP32 fills the LDS with 5 work-groups of 28 KB; 16-bit storage takes
+// 6, where nothing spills (76 to 80 VGPRs).  At 7 (72 VGPRs, 4 to 5 spilled) its
+// launches take the same time: 182.4 against 182.6 us at 28,416 work-groups,
+// 55.6 and 55.7 at 8,064, 38.1 and 38.0 at 4,320, 15.1 and 15.0 at 816.
 template <int ST, class OffT>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ST == 0 ? 5 : 6)))
 thermal_kernel(const LevelArgs* __restrict__ las, const CaseState* __restrict__ states,

@@ -29,8 +29,9 @@ def ramp_table(cfg, n_steps: int) -> np.ndarray:
 
 
 def default_waves(storage: int) -> int:
-    """The interior stream-collide kernel's default occupancy, as the library
-    picks it: 5 waves per SIMD for FP32 storage, 6 for 16-bit storage."""
+    """The stream-collide kernel's default occupancy, as the library picks it: 5
+    waves per SIMD for FP32 storage, 6 for 16-bit storage (whose launches of up
+    to 1,280 blocks run at 5 whatever is asked for)."""
     return 5 if storage == N.LB_STORAGE_FP32 else 6
 
 
@@ -123,7 +124,8 @@ class Engine:
 
     def set_options(self, graph: bool = True, schedule: int = N.LB_SCHED_LINEAR, waves: int | None = None) -> None:
         """Launch options (lb_engine_set_options); waves None: the storage's
-        default occupancy (5 waves per SIMD for FP32, 6 for 16-bit)."""
+        default occupancy (5 waves per SIMD for FP32, 6 for 16-bit).  16-bit
+        launches of up to 1,280 blocks run at 5 with either."""
         if waves is None:
             waves = default_waves(self.storage)
         self._check(self.lib.lb_engine_set_options(self._e, int(graph), int(schedule), int(waves)),
@@ -132,15 +134,16 @@ class Engine:
 
     def autotune(self, trial_steps: int = 2, candidates=None, margin: float = 0.03) -> dict:
         """Pick the launch options (graph replay, work-group schedule,
-        interior-kernel occupancy) by timing each on the attached cases.
-        Every option computes the same results, so the trial steps are real
-        steps of the cases.  The current options are timed first and kept
-        unless another candidate is faster by more than `margin`: trials on
-        a small mix are noisy, and the choice is reused for the mixes that
+        stream-collide occupancy) by timing each on the attached cases (where no
+        launch of a 16-bit mix has over 1,280 blocks, 5 and 6 waves are the same
+        kernel).  Every option computes the same results, so the trial steps
+        are real steps of the cases.  The current options are timed first and
+        kept unless another candidate is faster by more than `margin`: trials
+        on a small mix are noisy, and the choice is reused for the mixes that
         follow.  The default candidates leave out LB_SCHED_PERSISTENT, which
-        computes the same and measured 20-25 % slower on every mix tried (pass
-        it in `candidates` to include it).  Returns the chosen options and
-        the timings."""
+        computes the same and measured 1 to 24 % slower on mixes of 1 to 50 M
+        cells, 2 % faster on one of 1.3 M in 16 bits (pass it in `candidates` to
+        include it).  Returns the chosen options and the timings."""
         import itertools
         import time
         if candidates is None:
