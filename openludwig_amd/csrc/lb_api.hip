@@ -1042,8 +1042,10 @@ __global__ void stats_reduce_kernel(const double* __restrict__ part, int rows, d
 // idle context may stand behind everything that a busy one has queued (260 ms
 // behind 3,000 coarse steps of 1.3 M cells, for 2 of 16 contexts; as a copy
 // 0.1 ms), and an event behind a copy would too.  Otherwise the kernel: copies
-// need a quarter to a half longer for 1.3 to 52.5 M cells, and up to 0.1 ms
-// more for each of the smallest (55 k cells).
+// need a quarter to a half longer for 6 to 52.5 M cells, and up to 0.1 ms more
+// for each of the smallest (55 k cells).  Which one is settled as the download
+// begins; steps that another thread queues meanwhile can still come before the
+// kernel's next piece.
 // The pinned memory is 8 pieces of 4 MiB for the process, allocated when first
 // needed and given back with the last context.  A piece is held while it is
 // filled and read, never while a context's earlier work is waited for, so
